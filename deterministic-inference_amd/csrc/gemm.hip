@@ -23,6 +23,8 @@
 //     an optional fused greedy argmax.
 #include "common.h"
 
+#include <algorithm>
+
 namespace sid {
 namespace {
 
@@ -332,11 +334,13 @@ __device__ __forceinline__ void sstate_merge(SState& a, const SState& b, bool gr
   }
 }
 
-// Merge over the 16 lanes of a DPP row (xor butterfly; every lane ends with the same state).
-__device__ __forceinline__ void sstate_merge16(SState& a, bool greedy) {
+// Merge over the lanes that differ in the bits LO .. HI / 2 (xor butterfly; each of them ends
+// with the same state).
+template <int LO, int HI>
+__device__ __forceinline__ void sstate_merge_xor(SState& a, bool greedy) {
   const int lane = __lane_id();
 #pragma unroll
-  for (int mask = 1; mask < 16; mask <<= 1) {
+  for (int mask = LO; mask < HI; mask <<= 1) {
     SState b;
     b.m = lane_xor(a.m, mask);
     b.s = lane_xor(a.s, mask);
@@ -366,382 +370,551 @@ struct SampleIn {
   int64_t cand_rows;
 };
 
-// ---- large-M tiled GEMM (prefill) ---------------------------------------------------------
+// ---- pipelined tile GEMM (64 rows and more: prefill, verify passes, wide heads) ------------
 //
-// 128 x 128 output tile per 4-wave workgroup (wave (wm, wn): 64 x 64 = 4 x 4 MFMA blocks),
-// K streamed in 64-deep sub-tiles through double-buffered LDS (the next sub-tile's x and w
-// rows are loaded into registers while the current one's MFMAs run). Every output element
-// sees the canonical order: each 256-wide chunk accumulated from zero by 8 MFMA k-steps in
-// increasing k (two per sub-tile), the chunk sums left-folded c0 + c1 + ..., then + bias and
-// one rounding; the operand layout per MFMA is linear_kernel's. So the bits equal
-// sid_linear's for any M, while the tile reuse (each x row feeds 128 columns, each weight
-// row 128 rows) makes large M MFMA-bound instead of bound by re-reading operands.
-constexpr int TT_K = 64;
-// LDS row stride (bf16): 160 bytes. (Layout only; measured against 144 bytes, which
-// allows two workgroups per CU: 3-13% faster on prefill shapes M = 1024-8192, e.g. qkv at
-// M = 8192 95.6 -> 88.4 us, o at M = 4096 33.1 -> 29.3 us; an XOR-swizzled unpadded layout
-// measured the same as this padding.)
-constexpr int TT_KS = TT_K + 16;
-constexpr int TT_SUB_PER_CHUNK = KC / TT_K;
+// Persistent workgroups of WM x WN waves; wave (wm, wn) owns MB x NB MFMA blocks
+// (16 MB x 16 NB outputs) of a TM x TN tile. K streams in 64-deep sub-tiles through a ring of
+// ST LDS stages that buffer_load ... lds fills ST - 1 sub-tiles ahead, across tile boundaries
+// too, so a tile's first loads are in flight while the previous tile is stored. One barrier
+// per sub-tile: a wave that passes it has finished reading the stage about to be refilled, and
+// its wait count leaves the ST - 2 later sub-tiles in flight. Between two barriers the
+// fragment reads of one 32-deep k-step run beside the MFMAs of the k-step before it
+// (scheduling barriers keep that order), so neither LDS nor memory latency is exposed.
+//
+// LDS: a stage's rows are 128 bytes (64 bf16) without padding, 16-byte piece p of row q at
+// p ^ ((q >> 1) & 7): the DMA writes whole 1 KB runs (the permutation is on the global side,
+// inside one 128-byte line) and the fragment reads are conflict-free (SQ_LDS_BANK_CONFLICT
+// 0). Rows past M or N are dropped by the buffer range check (zeros); their outputs are not
+// stored. Weights are the MFMA's A operand, so a lane holds four consecutive columns of one
+// row and a tile is stored through LDS as whole 128-byte lines.
+//
+// Every output element keeps the canonical order: each 256-wide chunk accumulated from zero
+// by 8 MFMA k-steps in increasing k, the chunk sums left-folded in order, then + bias and one
+// rounding; products commute, so the bits are linear_kernel's for any M and any tile.
+//
+// Bound: MFMA issue and its power (random operands run ~20% below zeros); above that the
+// LDS fills, 47 bytes per clock and CU at the MFMA peak with 256 x 128 tiles. Two accumulator
+// sets (the chunk's and the fold's) limit a wave to 64 x 64 outputs. Measured against the
+// register-staged 128 x 128 tiles this replaced (us): 8192 x 4096 x 1024 96.4 -> 75.2,
+// 8192 x 6144 x 1024 129.5 -> 95.2, 8192 x 1024 x 3072 68.3 -> 46.0 (1.12 PFLOP/s),
+// 2048 x 1024 x 2048 17.9 -> 12.7, 777 x 1024 x 3072 21.4 -> 11.6; the vendor BLAS (not
+// batch-invariant) takes 57.6, 98.6 and 52.5 on the first three.
+//
+// EPI selects the epilogue: bf16 / fp32 y (+ bias); SwiGLU; the greedy or the seeded
+// sampler's statistics of the lm_head.
+constexpr int BK = 64;
+constexpr int SUBS = KC / BK;
+constexpr int EPI_Y = 0, EPI_SWIGLU = 1, EPI_ARGMAX = 2, EPI_SAMPLE = 3;
 
-// WM x WN waves; wave (wm, wn) owns MB x NB MFMA blocks = (16 MB) x (16 NB) outputs.
-// PF = 1: the next sub-tile is loaded into registers during the current one's MFMAs, and the
-// compiler schedules the loads among them (best when the grid fills the chip: the MFMAs
-// are the bound). PF = 2: a ring of two register buffers keeps two sub-tiles in flight,
-// issued at fixed points (best for grids of at most one workgroup per CU, where every
-// sub-tile's global-memory latency would otherwise be exposed). Same arithmetic either way.
-//
-// AM (greedy lm_head): the epilogue also keeps each row's best (bf16-rounded logit, column)
-// over the tile's columns, in argmax_better's order, and writes it to
-// best_val / best_idx [blockIdx.x][M] for argmax_finalize_kernel; y may then be null (no
-// logits written).
-//
-// SW (gate_up + SwiGLU, weights [gate rows | up rows] of inter rows each): the tile's first
-// NB/2 column blocks of each wave are gate rows and the last NB/2 the up rows of the same
-// inter columns, so a lane holds both values of its outputs; the epilogue writes
-// act[row][c] = silu_mul1(gate, up) of the bf16-rounded projections ([M, inter], the bits of
-// sid_silu_mul over sid_linear's output) and no projection.
-template <int WM, int WN, int MB, int NB, int PF, bool AM = false, bool SW = false,
-          bool SP = false>
-__global__ void __launch_bounds__(WM * WN * 64, (AM || SP) ? 4 : 1) linear_tiled_kernel(
-    const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ w,
-    const bf16_t* __restrict__ bias, void* __restrict__ y, int64_t M, int64_t N, int64_t K,
-    int out_fp32, float* __restrict__ best_val, int* __restrict__ best_idx, SampleIn sp) {
-  constexpr int TM = WM * MB * 16;
-  constexpr int TN = WN * NB * 16;
-  constexpr int THREADS = WM * WN * 64;
-  constexpr int LA = TM * (TT_K / 8) / THREADS;  // 16-byte x vectors per thread per sub-tile
-  constexpr int LB = TN * (TT_K / 8) / THREADS;
-  static_assert(LA * THREADS == TM * (TT_K / 8) && LB * THREADS == TN * (TT_K / 8), "tile");
-  __shared__ __align__(16) bf16_t sa[2][TM * TT_KS];
-  __shared__ __align__(16) bf16_t sb[2][TN * TT_KS];
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int lane = tid & 63;
+typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
+
+// Lane l's 16 bytes at srd base + voff + soff (range-checked) -> LDS byte lds + 16 l.
+__device__ __forceinline__ void dma16(uint32_t voff, u32x4_v srd, uint32_t soff, uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff),
+      "s"(srd), "s"(soff), "s"(lds)
+      : "memory", "m0");
+}
+
+// All but this wave's N newest loads have landed, its LDS reads are done, and every wave of
+// the workgroup got here.
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ u32x4_v raw_srd(const void* p, uint32_t bytes) {
+  const uint64_t a = reinterpret_cast<uintptr_t>(p);
+  return u32x4_v{static_cast<uint32_t>(a), static_cast<uint32_t>(a >> 32) & 0xffffu, bytes,
+                 0x00020000u};
+}
+__device__ __forceinline__ u32x4_v pick(bool c, const u32x4_v& a, const u32x4_v& b) {
+  return u32x4_v{c ? a[0] : b[0], c ? a[1] : b[1], c ? a[2] : b[2], c ? a[3] : b[3]};
+}
+
+// Output side of a launch. wide: y (and N) allow 16-byte stores. inter (SwiGLU): y is
+// [M][inter] and w holds inter gate rows, then inter up rows (N = 2 inter).
+struct TileOut {
+  void* y;
+  const bf16_t* bias;
+  int out_fp32;
+  int wide;
+  float* best_val;
+  int* best_idx;
+  SampleIn sp;
+};
+
+template <int WM, int WN, int MB, int NB, int ST>
+struct TileShape {
+  static constexpr int NW = WM * WN;
+  static constexpr int TM = WM * MB * 16;
+  static constexpr int TN = WN * NB * 16;
+  static constexpr int STAGE = (TM + TN) * BK * 2;
+  static constexpr int SCRATCH = NW * 2048;  // epilogue: 2 KB per wave
+  static constexpr int LDS = ST * STAGE + SCRATCH;
+};
+
+template <int WM, int WN, int MB, int NB, int ST, int OCC, int EPI>
+__global__ void __launch_bounds__(WM * WN * 64, OCC) linear_tile_kernel(
+    const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ w, int M, int N, int K,
+    int mt, int nt, TileOut out) {
+  using S = TileShape<WM, WN, MB, NB, ST>;
+  constexpr int NW = S::NW, TM = S::TM, TN = S::TN, STAGE = S::STAGE;
+  constexpr int PA = TM / 8 / NW, PB = TN / 8 / NW;  // 1 KB pieces a wave loads per sub-tile
+  constexpr int PER = PA + PB;
+  static_assert(PA * 8 * NW == TM && PB * 8 * NW == TN && NB % 2 == 0, "tile");
+  static_assert(EPI != EPI_SWIGLU || (NW / 2) % NB == 0, "a wave's w pieces are all gate or all up");
+  extern __shared__ __align__(1024) char lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   const int r = lane & 15;
   const int g = lane >> 4;
   const int wm = wave / WN;
   const int wn = wave % WN;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * TN;
-  const int64_t m0 = static_cast<int64_t>(blockIdx.y) * TM;
+  const int tiles = mt * nt;
+  const int nsub = K / BK;  // a multiple of 4, at least ST - 1 (the host's choice of shape)
+  const int nch = K / KC;
+  const uint32_t lds0 = static_cast<uint32_t>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds));
 
-  // Sub-tile loads (8 vectors of 16 bytes per 64-deep row). Rows past M (x) or N (w) are
-  // clamped to the last valid row; their results are dropped.
-  const bf16_t* xrow[LA];
-  const bf16_t* wrow[LB];
-  int arow[LA], avec[LA], brow[LB], bvec[LB];
+  // Tile order: bands of 4 row tiles, rows fastest, so the tiles in flight share x and w
+  // rows; XCD k (workgroups k mod 8) takes a contiguous eighth of each round of the grid.
+  auto tile_mn = [&](int t, int& tm, int& tn) {
+    constexpr int BAND = 4;
+    const int band = t / (BAND * nt);
+    const int rem = t - band * BAND * nt;
+    const int rows = min(BAND, mt - band * BAND);
+    tn = rem / rows;
+    tm = band * BAND + rem - tn * rows;
+  };
+  const int grid = gridDim.x;
+  int t = blockIdx.x;
+  if (grid % 8 == 0) t = (blockIdx.x % 8) * (grid / 8) + blockIdx.x / 8;
+
+  // Loads: piece p = wave + NW i is rows 8p .. 8p+7 of the stage's x (w) part, lane l row
+  // l / 8, global 16-byte piece (l % 8) ^ swizzle. SwiGLU: LDS row j of the w part is, in
+  // wave column block order, a gate row (first NB / 2 blocks) or the up row of the same
+  // output column; a piece lies in one block, so the wave loads only gate or only up rows.
+  uint32_t voa[PA], vob[PB];
 #pragma unroll
-  for (int i = 0; i < LA; ++i) {
-    const int v = tid + THREADS * i;
-    arow[i] = v >> 3;
-    avec[i] = v & 7;
-    xrow[i] = x + min<int64_t>(m0 + arow[i], M - 1) * ldx + avec[i] * 8;
+  for (int i = 0; i < PA; ++i) {
+    const int row = 8 * (wave + NW * i) + (lane >> 3);
+    voa[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(2 * ldx) +
+             16u * ((lane & 7) ^ ((row >> 1) & 7));
   }
 #pragma unroll
-  for (int i = 0; i < LB; ++i) {
-    const int v = tid + THREADS * i;
-    brow[i] = v >> 3;
-    bvec[i] = v & 7;
-    int64_t wr = n0 + brow[i];
-    if constexpr (SW) {  // LDS row j = wave column block's row: gate or up row of column c
-      static_assert(NB % 2 == 0, "SwiGLU tiles pair gate and up column blocks");
-      const int jw = brow[i] / (NB * 16);
-      const int jb = (brow[i] / 16) % NB;
-      const int64_t c = blockIdx.x * (TN / 2) + jw * (NB / 2) * 16 + (jb % (NB / 2)) * 16 +
-                        (brow[i] % 16);
-      wr = jb < NB / 2 ? c : N / 2 + c;
+  for (int i = 0; i < PB; ++i) {
+    const int row = 8 * (wave + NW * i) + (lane >> 3);
+    int src = row;
+    if constexpr (EPI == EPI_SWIGLU) {
+      const int block = row / 16;
+      src = (block / NB) * (NB / 2) * 16 + (block % NB % (NB / 2)) * 16 + row % 16;
     }
-    wrow[i] = w + min<int64_t>(wr, N - 1) * K + bvec[i] * 8;
+    vob[i] = static_cast<uint32_t>(src) * static_cast<uint32_t>(2 * K) +
+             16u * ((lane & 7) ^ ((row >> 1) & 7));
   }
-  static_assert(PF == 1 || PF == 2 || PF == 4, "PF must divide the 4 sub-tiles of a chunk");
-  bf16x8_v ra[PF][LA], rb[PF][LB];
-  auto load_sub = [&](int kt, bf16x8_v (&da)[LA], bf16x8_v (&db)[LB]) {
-    const int64_t k0 = static_cast<int64_t>(kt) * TT_K;
-#pragma unroll
-    for (int i = 0; i < LA; ++i) da[i] = ld_frag(xrow[i] + k0);
-#pragma unroll
-    for (int i = 0; i < LB; ++i) db[i] = ld_frag(wrow[i] + k0);
+  u32x4_v sa, sb, na, nb;  // this tile's and the next one's buffers
+  auto tile_srd = [&](int tt, u32x4_v& a, u32x4_v& b) {
+    int tm, tn;
+    const bool ok = tt < tiles;  // no next tile: every load is out of range
+    tile_mn(ok ? tt : 0, tm, tn);
+    const int m0 = tm * TM;
+    a = raw_srd(x + static_cast<int64_t>(m0) * ldx,
+                ok ? static_cast<uint32_t>(min(TM, M - m0)) * static_cast<uint32_t>(2 * ldx) : 0u);
+    int n0 = tn * TN, rows = min(TN, N - n0);
+    if constexpr (EPI == EPI_SWIGLU) {
+      const int inter = N / 2;
+      n0 = tn * (TN / 2);
+      rows = min(TN / 2, inter - n0);
+      if ((wave / 2) % NB >= NB / 2) n0 += inter;
+    }
+    b = raw_srd(w + static_cast<int64_t>(n0) * K,
+                ok ? static_cast<uint32_t>(rows) * static_cast<uint32_t>(2 * K) : 0u);
   };
-  auto store_sub = [&](int buf, const bf16x8_v (&da)[LA], const bf16x8_v (&db)[LB]) {
-#pragma unroll
-    for (int i = 0; i < LA; ++i)
-      *reinterpret_cast<bf16x8_v*>(&sa[buf][arow[i] * TT_KS + avec[i] * 8]) = da[i];
-#pragma unroll
-    for (int i = 0; i < LB; ++i)
-      *reinterpret_cast<bf16x8_v*>(&sb[buf][brow[i] * TT_KS + bvec[i] * 8]) = db[i];
+  uint32_t lbuf = 0;  // the stage that the next loads fill
+  uint32_t cbuf = 0;  // the stage being multiplied
+  auto next_stage = [&](uint32_t b) { return b + STAGE == ST * STAGE ? 0u : b + STAGE; };
+  auto load_piece = [&](int i, const u32x4_v& a, const u32x4_v& b, uint32_t koff) {
+    const uint32_t dst = lds0 + lbuf + 1024u * wave;
+    if (i < PA) {
+      dma16(voa[i], a, koff, dst + 1024u * NW * i);
+    } else {
+      dma16(vob[i - PA], b, koff, dst + TM * 128u + 1024u * NW * (i - PA));
+    }
   };
+  tile_srd(t, sa, sb);
+#pragma unroll
+  for (int s = 0; s < ST - 1; ++s) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) load_piece(i, sa, sb, 128u * s);
+    lbuf = next_stage(lbuf);
+  }
 
+  const uint32_t abase = (wm * MB * 16 + r) * 128 + 16 * (g ^ ((r >> 1) & 7));
+  const uint32_t bbase = TM * 128 + (wn * NB * 16 + r) * 128 + 16 * (g ^ ((r >> 1) & 7));
+  bf16x8_v fa[2][MB], fb[2][NB];
   f32x4_v acc[MB][NB], tot[MB][NB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4_v{0.0f, 0.0f, 0.0f, 0.0f};
-  }
-  // One sub-tile's MFMAs out of LDS buffer `cur`, and the fold at the end of a chunk.
-  auto mma_sub = [&](int cur) {
-#pragma unroll
-    for (int s = 0; s < TT_K / KSTEP; ++s) {
-      bf16x8_v af[MB], bfv[NB];
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-        af[mb] = *reinterpret_cast<const bf16x8_v*>(
-            &sa[cur][(MB * 16 * wm + 16 * mb + r) * TT_KS + KSTEP * s + 8 * g]);
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-        bfv[nb] = *reinterpret_cast<const bf16x8_v*>(
-            &sb[cur][(NB * 16 * wn + 16 * nb + r) * TT_KS + KSTEP * s + 8 * g]);
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[mb], bfv[nb], acc[mb][nb], 0, 0, 0);
-      }
+  auto read_frag = [&](int s, int i) {
+    if (i < NB) {
+      fb[s][i] = *reinterpret_cast<const bf16x8_v*>(lds + cbuf + (bbase ^ (64u * s)) + 2048 * i);
+    } else {
+      fa[s][i - NB] =
+          *reinterpret_cast<const bf16x8_v*>(lds + cbuf + (abase ^ (64u * s)) + 2048 * (i - NB));
     }
   };
-  auto fold = [&](bool first) {  // chunk complete: fold, restart
+  // Half a sub-tile: the fragments of its k-step s are read while the k-step before is
+  // multiplied (mul), two MFMAs per read, the next stage's loads (load) among them. zero:
+  // the products start a chunk. fold: first fold the block's finished chunk sum into tot
+  // (keep = -0 for a tile's first chunk: tot is +0 then, and -0 * 0 + acc is acc bit for bit).
+  constexpr int NR = MB + NB, NM = MB * NB;
+  auto half = [&](int s, bool mul, bool zero, bool fold, float keep, bool load, const u32x4_v& a,
+                  const u32x4_v& b, uint32_t koff) {
+    int reads = 0, loads = 0;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
+    for (int k = 0; k < NM; ++k) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        if (first) {
-          tot[mb][nb] = acc[mb][nb];
-        } else {
+      for (int q = 0; q < 2; ++q) {
+        const int want = ((k + 2) * NR * 4 + 3 * NM - 1) / (3 * NM);  // all in 3/4 of the MFMAs
+        if (reads < NR && reads < want) read_frag(s, reads++);
+      }
+      if (load && loads < PER) {
+        load_piece(loads, a, b, koff);
+        ++loads;
+      }
+      if (mul) {
+        const int i = k / NB, j = k % NB;
+        if (fold) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) tot[mb][nb][i] += acc[mb][nb][i];
+          for (int e = 0; e < 4; ++e)
+            tot[i][j][e] = __builtin_fmaf(tot[i][j][e], keep, acc[i][j][e]);
         }
-        acc[mb][nb] = f32x4_v{0.0f, 0.0f, 0.0f, 0.0f};
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            fb[1 - s][j], fa[1 - s][i], zero ? f32x4_v{0.0f, 0.0f, 0.0f, 0.0f} : acc[i][j], 0, 0,
+            0);
+        if (k % 2 == 1) __builtin_amdgcn_sched_barrier(0);
       }
     }
+#pragma unroll
+    for (; reads < NR; ++reads) read_frag(s, reads);
+    if (load) {
+#pragma unroll
+      for (; loads < PER; ++loads) load_piece(loads, a, b, koff);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   };
 
-  const int nsub = static_cast<int>(K / TT_K);  // a multiple of 4 (K is a multiple of 256)
-  if constexpr (PF == 1) {
-    load_sub(0, ra[0], rb[0]);
-    store_sub(0, ra[0], rb[0]);
-    __syncthreads();
-    for (int kt = 0; kt < nsub; ++kt) {
-      const int cur = kt & 1;
-      if (kt + 1 < nsub) load_sub(kt + 1, ra[0], rb[0]);
-      mma_sub(cur);
-      if (kt % TT_SUB_PER_CHUNK == TT_SUB_PER_CHUNK - 1) fold(kt < TT_SUB_PER_CHUNK);
-      if (kt + 1 < nsub) {
-        store_sub(cur ^ 1, ra[0], rb[0]);
-        __syncthreads();
+  while (t < tiles) {
+    const int t_next = t + grid;
+    tile_srd(t_next, na, nb);
+    for (int c = 0; c < nch; ++c) {
+      const float keep = c == 1 ? -0.0f : 1.0f;
+#pragma unroll
+      for (int j = 0; j < SUBS; ++j) {
+        wait_barrier<PER * (ST - 2)>();
+        // Load sub-tile q + ST - 1 of the stream into the stage read last before the barrier.
+        const int sub = SUBS * c + j + ST - 1;
+        const bool next = sub >= nsub;
+        const u32x4_v a = pick(next, na, sa);
+        const u32x4_v b = pick(next, nb, sb);
+        const uint32_t koff = 128u * (next ? sub - nsub : sub);
+        if (j == 0 && c == 0) {
+          half(0, false, false, false, 1.0f, true, a, b, koff);
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int q = 0; q < NB; ++q) tot[mb][q] = f32x4_v{0.0f, 0.0f, 0.0f, 0.0f};
+          half(1, true, true, false, 1.0f, false, a, b, 0);
+        } else {
+          half(0, true, false, false, 1.0f, true, a, b, koff);
+          half(1, true, j == 0, j == 0, keep, false, a, b, 0);
+        }
+        lbuf = next_stage(lbuf);
+        cbuf = next_stage(cbuf);
       }
     }
-  } else {
-    // One 256-wide chunk (4 sub-tiles) per outer iteration. Sub-tile t lives in register
-    // slot t % PF until it is stored to LDS buffer t & 1. The loads PF sub-tiles ahead are
-    // unconditional (indices clamped to the last sub-tile, whose repeats are stored but
-    // never read), so the loop is straight-line and each store waits only for its own
-    // slot's loads; a scheduling barrier keeps each batch of loads where it is issued.
-    load_sub(0, ra[0], rb[0]);
-    store_sub(0, ra[0], rb[0]);
+    // The last k-step's products and the last fold.
+    const float keep = nch == 1 ? -0.0f : 1.0f;
 #pragma unroll
-    for (int p = 1; p <= PF; ++p) load_sub(min(p, nsub - 1), ra[p % PF], rb[p % PF]);
-    __syncthreads();
-    const int nch = nsub / TT_SUB_PER_CHUNK;
-    for (int c = 0; c < nch; ++c) {
+    for (int i = 0; i < MB; ++i) {
 #pragma unroll
-      for (int j = 0; j < TT_SUB_PER_CHUNK; ++j) {
-        const int kt = c * TT_SUB_PER_CHUNK + j;
-        const int cur = j & 1;  // kt & 1
-        mma_sub(cur);
-        if (j == TT_SUB_PER_CHUNK - 1) fold(c == 0);
-        const int slot = (j + 1) % PF;  // sub-tile kt + 1 (4 c is a multiple of PF)
-        store_sub(cur ^ 1, ra[slot], rb[slot]);
-        __syncthreads();
-        load_sub(min(kt + 1 + PF, nsub - 1), ra[slot], rb[slot]);
+      for (int j = 0; j < NB; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[1][j], fa[1][i], acc[i][j], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          tot[i][j][e] = __builtin_fmaf(tot[i][j][e], keep, acc[i][j][e]);
+      }
+    }
+    // Lane: row 16 i + r of the wave's rows, columns 16 j + 4 g .. +3. (el is the lane,
+    // opaque to the compiler: addresses derived from it are not kept through the main loop.)
+    int el = lane;
+    asm volatile("" : "+v"(el));
+    const int er = el & 15, eg = el >> 4;
+    int tm, tn;
+    tile_mn(t, tm, tn);
+    const int row0 = tm * TM + wm * MB * 16;
+    char* scratch = lds + ST * STAGE;
+    if constexpr (EPI == EPI_Y || EPI == EPI_SWIGLU) {
+      // One row block (IB of them where a store covers more than 16 rows) at a time. bf16
+      // goes through the wave's 2 KB of scratch, so that a store covers whole 32 CB-byte row
+      // segments (direct 8-byte stores: 8192 x 6144 104.9 -> 95.2 us).
+      constexpr int CB = EPI == EPI_SWIGLU ? NB / 2 : NB;  // column blocks written per wave
+      constexpr int PPR = 2 * CB;                          // 16-byte pieces per staged row
+      constexpr int RPS = 64 / PPR;                        // rows per store
+      constexpr int IB = RPS > 16 ? RPS / 16 : 1;
+      static_assert(MB % IB == 0 && 16 * IB * 16 * PPR <= 2048, "store staging");
+      const int ncols = EPI == EPI_SWIGLU ? N / 2 : N;
+      const int col0 = (tn * WN + wn) * CB * 16;
+      char* st = scratch + wave * 2048;
+#pragma unroll
+      for (int i0 = 0; i0 < MB; i0 += IB) {
+#pragma unroll
+        for (int i = i0; i < i0 + IB; ++i) {
+          const int64_t row = row0 + 16 * i + er;
+#pragma unroll
+          for (int j = 0; j < CB; ++j) {
+            const int col = col0 + 16 * j + 4 * eg;
+            f32x4_v v = tot[i][j];
+            if constexpr (EPI == EPI_SWIGLU) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                v[e] = silu_mul1(round_bf16(v[e]), round_bf16(tot[i][j + NB / 2][e]));
+            } else if (out.bias != nullptr && col < N) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[e] += bf16_to_f32(out.bias[col + e]);
+            }
+            const u32x2_v u = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            if (out.wide && !out.out_fp32) {
+              *reinterpret_cast<u32x2_v*>(st + (16 * (i - i0) + er) * (16 * PPR) +
+                                          16 * ((2 * j + (eg >> 1)) ^ (er & (PPR - 1))) +
+                                          8 * (eg & 1)) = u;
+            } else if (row < M && col < ncols) {
+              if (out.out_fp32) {
+                float* y = static_cast<float*>(out.y) + row * ncols + col;
+                const f32x4_v q = {bf16_lo(u[0]), bf16_hi(u[0]), bf16_lo(u[1]), bf16_hi(u[1])};
+                if (out.wide) {
+                  *reinterpret_cast<f32x4_v*>(y) = q;
+                } else {
+#pragma unroll
+                  for (int e = 0; e < 4; ++e) y[e] = q[e];
+                }
+              } else {
+                bf16_t* y = static_cast<bf16_t*>(out.y) + row * ncols + col;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  y[e] = static_cast<bf16_t>(u[e / 2] >> (16 * (e % 2)));
+              }
+            }
+          }
+        }
+        if (out.wide && !out.out_fp32) {
+          bf16_t* y = static_cast<bf16_t*>(out.y);
+          const int pp = el % PPR;
+#pragma unroll
+          for (int q = 0; q < 16 * IB / RPS; ++q) {
+            const int lr = RPS * q + el / PPR;
+            const u32x4_v u = *reinterpret_cast<const u32x4_v*>(
+                st + lr * (16 * PPR) + 16 * (pp ^ (lr & (PPR - 1))));
+            const int64_t row = row0 + 16 * i0 + lr;
+            const int col = col0 + 8 * pp;
+            if (row < M && col < ncols) *reinterpret_cast<u32x4_v*>(y + row * ncols + col) = u;
+          }
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
-    }
-  }
-
-  // Lane holds rows 16*mb + 4*g + i, column 16*nb + r of the wave's block.
-  if constexpr (SW) {
-    const int64_t inter = N / 2;
+    } else {
+      // lm_head epilogues: each lane's best (EPI_ARGMAX) or sampler state (EPI_SAMPLE) of a
+      // row over its 4 NB columns in increasing order (logits written as fp32 when y is
+      // given), merged over the 4 lanes of the row, then over the WN waves of the row band in
+      // wave order through LDS: one record per (column tile, row).
+      float* s_f = reinterpret_cast<float*>(scratch);
+      static_assert(6 * WN * TM * 4 <= S::SCRATCH, "statistics exceed the scratch");
+      int* s_i = reinterpret_cast<int*>(s_f + 5 * WN * TM);
+      const int col0 = (tn * WN + wn) * NB * 16;
 #pragma unroll
-    for (int nb = 0; nb < NB / 2; ++nb) {
-      const int64_t col = blockIdx.x * (TN / 2) + wn * (NB / 2) * 16 + 16 * nb + r;
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int64_t row = m0 + MB * 16 * wm + 16 * mb + 4 * g + i;
-          if (row >= M) continue;
-          const float gv = round_bf16(tot[mb][nb][i]);
-          const float uv = round_bf16(tot[mb][nb + NB / 2][i]);
-          static_cast<bf16_t*>(y)[row * inter + col] = f32_to_bf16(silu_mul1(gv, uv));
+      for (int i = 0; i < MB; ++i) {
+        const int lr = wm * MB * 16 + 16 * i + er;
+        const int64_t row = static_cast<int64_t>(tm) * TM + lr;
+        const bool row_ok = row < M;
+        float temp = 0.0f;
+        uint32_t h = 0;
+        if constexpr (EPI == EPI_SAMPLE) {
+          const int64_t rc = row_ok ? row : M - 1;
+          temp = out.sp.temps[rc];
+          h = gumbel_row(out.sp.seeds[rc], out.sp.positions[rc]);
         }
-      }
-    }
-  } else if constexpr (SP) {
-    // Sampler epilogue, one row block at a time: each lane's statistics over its columns
-    // (logits written as fp32 when y is given), merged over the 16 column lanes of a row,
-    // then over the WN waves of a row band in wave order through LDS (the x tile buffer,
-    // free once every wave is past its last MFMA); one record per (column tile, row).
-    float* s_f = reinterpret_cast<float*>(&sa[0][0]);  // [5][WN][TM] floats, then [WN][TM] ints
-    int* s_i = reinterpret_cast<int*>(s_f + 5 * WN * TM);
-    static_assert(6 * WN * TM * 4 <= TM * TT_KS * 2, "sampler scratch exceeds the x tile");
-    __syncthreads();
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int lr = MB * 16 * wm + 16 * mb + 4 * g + i;
-        const int64_t row = m0 + lr;
-        const int64_t rc = min<int64_t>(row, M - 1);
-        const float t = sp.temps[rc];
-        const uint32_t h = gumbel_row(sp.seeds[rc], sp.positions[rc]);
         SState a = sstate_empty();
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          const int64_t col = n0 + NB * 16 * wn + 16 * nb + r;
-          if (col >= N || row >= M) continue;
-          const float vr = round_bf16(tot[mb][nb][i]);
-          if (y != nullptr) static_cast<float*>(y)[row * N + col] = vr;
-          sstate_add(a, vr, static_cast<int>(col), t, h);
+        for (int j = 0; j < NB; ++j) {
+          const int col = col0 + 16 * j + 4 * eg;
+          if (col >= N || !row_ok) continue;
+          f32x4_v q;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float v = tot[i][j][e];
+            if (EPI == EPI_ARGMAX && out.bias != nullptr) v += bf16_to_f32(out.bias[col + e]);
+            q[e] = round_bf16(v);
+            if constexpr (EPI == EPI_SAMPLE) {
+              sstate_add(a, q[e], col + e, temp, h);
+            } else if (argmax_better(q[e], col + e, a.v1, a.i1)) {
+              a.v1 = q[e];
+              a.i1 = col + e;
+            }
+          }
+          if (out.y != nullptr) {
+            float* y = static_cast<float*>(out.y) + row * N + col;
+            if (out.wide) {
+              *reinterpret_cast<f32x4_v*>(y) = q;
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) y[e] = q[e];
+            }
+          }
         }
-        sstate_merge16(a, !(t > 0.0f));
-        if (r == 0) {
+        sstate_merge_xor<16, 64>(a, EPI == EPI_ARGMAX || !(temp > 0.0f));
+        if (eg == 0) {
           const int o = wn * TM + lr;
-          s_f[o] = a.m;
-          s_f[WN * TM + o] = a.s;
           s_f[2 * WN * TM + o] = a.v1;
-          s_f[3 * WN * TM + o] = a.x1;
-          s_f[4 * WN * TM + o] = a.v2;
           s_i[o] = a.i1;
+          if constexpr (EPI == EPI_SAMPLE) {
+            s_f[o] = a.m;
+            s_f[WN * TM + o] = a.s;
+            s_f[3 * WN * TM + o] = a.x1;
+            s_f[4 * WN * TM + o] = a.v2;
+          }
         }
       }
-    }
-    __syncthreads();
-    for (int lr = tid; lr < TM; lr += THREADS) {
-      const int64_t row = m0 + lr;
-      if (row >= M) continue;
-      const bool greedy = !(sp.temps[row] > 0.0f);
-      SState a = sstate_empty();
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      for (int lr = threadIdx.x; lr < TM; lr += NW * 64) {
+        const int64_t row = static_cast<int64_t>(tm) * TM + lr;
+        if (row >= M) continue;
+        SState a = sstate_empty();
+        const bool greedy = EPI == EPI_ARGMAX || !(out.sp.temps[row] > 0.0f);
 #pragma unroll
-      for (int q = 0; q < WN; ++q) {
-        const int o = q * TM + lr;
-        const SState b{s_f[o], s_f[WN * TM + o], s_f[2 * WN * TM + o], s_f[3 * WN * TM + o],
-                       s_f[4 * WN * TM + o], s_i[o]};
-        if (q == 0) {
-          a = b;
-        } else {
-          sstate_merge(a, b, greedy);
-        }
-      }
-      sstate_store(sp.st, static_cast<int64_t>(blockIdx.x) * sp.cand_rows + row, a);
-    }
-  } else if constexpr (!AM) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      const int64_t col = n0 + NB * 16 * wn + 16 * nb + r;
-      if (col >= N) continue;
-      const float bv = bias != nullptr ? bf16_to_f32(bias[col]) : 0.0f;
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int64_t row = m0 + MB * 16 * wm + 16 * mb + 4 * g + i;
-          if (row >= M) continue;
-          float v = tot[mb][nb][i];
-          if (bias != nullptr) v += bv;
-          if (out_fp32) {
-            static_cast<float*>(y)[row * N + col] = round_bf16(v);
+        for (int q = 0; q < WN; ++q) {
+          const int o = q * TM + lr;
+          SState b = sstate_empty();
+          b.v1 = s_f[2 * WN * TM + o];
+          b.i1 = s_i[o];
+          if constexpr (EPI == EPI_SAMPLE) {
+            b.m = s_f[o];
+            b.s = s_f[WN * TM + o];
+            b.x1 = s_f[3 * WN * TM + o];
+            b.v2 = s_f[4 * WN * TM + o];
+          }
+          if (q == 0) {
+            a = b;
           } else {
-            static_cast<bf16_t*>(y)[row * N + col] = f32_to_bf16(v);
+            sstate_merge(a, b, greedy);
           }
+        }
+        if constexpr (EPI == EPI_SAMPLE) {
+          sstate_store(out.sp.st, static_cast<int64_t>(tn) * out.sp.cand_rows + row, a);
+        } else {
+          out.best_val[static_cast<int64_t>(tn) * M + row] = a.v1;
+          out.best_idx[static_cast<int64_t>(tn) * M + row] = a.i1;
         }
       }
     }
+    t = t_next;
+    sa = na;
+    sb = nb;
+  }
+  // Loads issued past the last sub-tile (out of range) still write LDS: they must land
+  // before the workgroup's LDS is given back.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// Compute units of the current device.
+int cu_count() {
+  static int count[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (count[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      n = 256;
+    count[dev] = n;
+  }
+  return count[dev];
+}
+
+template <int WM, int WN, int MB, int NB, int ST, int OCC, int PER_CU, int EPI>
+void launch_tile(const void* x, int64_t ldx, const void* w, int64_t m, int64_t n, int64_t k,
+                 const TileOut& out, hipStream_t s) {
+  using S = TileShape<WM, WN, MB, NB, ST>;
+  static_assert(S::LDS * PER_CU <= 160 * 1024, "LDS");
+  auto kern = linear_tile_kernel<WM, WN, MB, NB, ST, OCC, EPI>;
+  static bool attr_set = false;
+  if (!attr_set) {
+    hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                        hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
+    attr_set = true;
+  }
+  const int mt = static_cast<int>((m + S::TM - 1) / S::TM);
+  const int nt = static_cast<int>((n + S::TN - 1) / S::TN);
+  const int grid = static_cast<int>(
+      std::min<int64_t>(static_cast<int64_t>(mt) * nt, static_cast<int64_t>(cu_count()) * PER_CU));
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(S::NW * 64), S::LDS, s, (const bf16_t*)x, ldx,
+                     (const bf16_t*)w, (int)m, (int)n, (int)k, mt, nt, out);
+}
+// The tile shapes, and the one a problem takes: the cheapest by a model of the main loop, the
+// grid's rounds times a round's time per 64-deep sub-tile (ns; identical bits, so this is
+// only speed). Measured with K = 1024-3072, M = 100-8420: 256 x 128 970 and 128 x 128 500 (all
+// CUs busy), 128 x 64 330, 64 x 64 210 while every CU has at most one tile and 380 with two.
+// Large problems are at the MFMA / power bound with the first two, small ones at the memory
+// round trips of few workgroups, which smaller tiles spread over more CUs: 777 x 1024 x 3072
+// 20.7 (128 x 128) vs 11.6 us (64 x 64), 2048 x 1024 x 2048 15.1 (128 x 128) vs 12.7 (128 x
+// 64), 8420 x 1024 x 2048 50.5 (256 x 128, a second round for 8 tiles) vs 43.7 (128 x 128).
+template <int EPI>
+void launch_tiles(const void* x, int64_t ldx, const void* w, int64_t m, int64_t n, int64_t k,
+                  const TileOut& out, hipStream_t s) {
+  if constexpr (EPI == EPI_ARGMAX || EPI == EPI_SAMPLE) {
+    // 128-column tiles: the candidate grouping of the lm_head epilogues
+    launch_tile<4, 2, 2, 4, 4, 2, 1, EPI>(x, ldx, w, m, n, k, out, s);
   } else {
-    // Greedy epilogue, one row block at a time (few live registers: the kernel keeps its
-    // occupancy): each lane's best over its columns (logits written as fp32 when y is
-    // given), then over the 16 column lanes of each row, then over the WN waves of a row
-    // band through LDS (the x tile buffer, free once every wave is past its last MFMA).
-    float* s_v = reinterpret_cast<float*>(&sa[0][0]);
-    int* s_i = reinterpret_cast<int*>(s_v + WN * TM);
-    static_assert(2 * WN * TM * 4 <= TM * TT_KS * 2, "argmax scratch exceeds the x tile");
-    __syncthreads();
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int64_t row = m0 + MB * 16 * wm + 16 * mb + 4 * g + i;
-        float v = -INFINITY;
-        int ix = 0x7fffffff;
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          const int64_t col = n0 + NB * 16 * wn + 16 * nb + r;
-          if (col >= N || row >= M) continue;
-          float t = tot[mb][nb][i];
-          if (bias != nullptr) t += bf16_to_f32(bias[col]);
-          const float vr = round_bf16(t);
-          if (y != nullptr) static_cast<float*>(y)[row * N + col] = vr;
-          if (argmax_better(vr, static_cast<int>(col), v, ix)) {
-            v = vr;
-            ix = static_cast<int>(col);
-          }
-        }
-#pragma unroll
-        for (int mask = 1; mask < 16; mask <<= 1) {
-          const float ov = lane_xor(v, mask);
-          const int oi = __builtin_amdgcn_ds_bpermute((lane ^ mask) << 2, ix);
-          if (argmax_better(ov, oi, v, ix)) {
-            v = ov;
-            ix = oi;
-          }
-        }
-        if (r == 0) {
-          const int lr = MB * 16 * wm + 16 * mb + 4 * g + i;
-          s_v[wn * TM + lr] = v;
-          s_i[wn * TM + lr] = ix;
-        }
-      }
-    }
-    __syncthreads();
-    for (int lr = tid; lr < TM; lr += THREADS) {
-      float v = s_v[lr];
-      int ix = s_i[lr];
-#pragma unroll
-      for (int q = 1; q < WN; ++q) {
-        if (argmax_better(s_v[q * TM + lr], s_i[q * TM + lr], v, ix)) {
-          v = s_v[q * TM + lr];
-          ix = s_i[q * TM + lr];
-        }
-      }
-      const int64_t row = m0 + lr;
-      if (row < M) {
-        best_val[static_cast<int64_t>(blockIdx.x) * M + row] = v;
-        best_idx[static_cast<int64_t>(blockIdx.x) * M + row] = ix;
-      }
+    const int64_t cus = cu_count();
+    auto tiles = [&](int tm, int tn) { return ((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
+    auto rounds = [&](int64_t t, int64_t slots) { return (t + slots - 1) / slots; };
+    const int64_t t64 = tiles(64, 64);
+    const int64_t cost[4] = {970 * rounds(tiles(256, 128), cus), 500 * rounds(tiles(128, 128), cus),
+                             330 * rounds(tiles(128, 64), cus),
+                             t64 <= cus ? 210 : 380 * rounds(t64, 2 * cus)};
+    int best = 0;
+    for (int i = 1; i < 4; ++i)
+      if (cost[i] < cost[best]) best = i;
+    switch (best) {
+      case 0: launch_tile<4, 2, 4, 4, 3, 2, 1, EPI>(x, ldx, w, m, n, k, out, s); break;
+      case 1: launch_tile<4, 2, 2, 4, 4, 2, 1, EPI>(x, ldx, w, m, n, k, out, s); break;
+      case 2: launch_tile<4, 2, 2, 2, 5, 2, 1, EPI>(x, ldx, w, m, n, k, out, s); break;
+      default: launch_tile<2, 2, 2, 2, 4, 1, 2, EPI>(x, ldx, w, m, n, k, out, s); break;
     }
   }
 }
 
-template <int WM, int WN, int MB, int NB, int PF, bool AM = false, bool SW = false,
-          bool SP = false>
-void launch_tiled(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t m,
-                  int64_t n, int64_t k, int out_fp32, hipStream_t s, float* best_val = nullptr,
-                  int* best_idx = nullptr, SampleIn sp = SampleIn{}) {
-  constexpr int TM = WM * MB * 16, TN = WN * NB * 16;
-  const dim3 grid((unsigned)((n + TN - 1) / TN), (unsigned)((m + TM - 1) / TM));
-  hipLaunchKernelGGL((linear_tiled_kernel<WM, WN, MB, NB, PF, AM, SW, SP>), grid,
-                     dim3(WM * WN * 64), 0, s, (const bf16_t*)x, ldx, (const bf16_t*)w,
-                     (const bf16_t*)bias, y, m, n, k, out_fp32, best_val, best_idx, sp);
+// Sizes whose tile offsets fit the kernel's 32-bit buffer ranges and indices.
+bool tiles_fit(int64_t ldx, int64_t m, int64_t n, int64_t k) {
+  return ldx < (1ll << 22) && k < (1ll << 22) && m < (1ll << 31) && n < (1ll << 30);
 }
 
-// sid_linear takes the tiled kernel from this many rows up: 8 waves (4 x 2), each 32 x 64
-// outputs (a 128 x 128 tile), or 32 x 32 (128 x 64) when 128 x 128 tiles would leave fewer
-// than two workgroups per CU. (Measured on prefill shapes: 25-29% of the bf16 MFMA peak at
-// M >= 2048 vs 8% for the 64-row-group kernel; 4 waves of 64 x 64 held both accumulator
-// sets in AGPRs at one wave per SIMD and reached 13%. From 64 rows it also beats the 64-row-
-// group kernel on the decode shapes, weights from HBM, consumer included: qkv at 128 rows
-// 15.8 vs 22.1 us, o 19.3 vs 33.0, down 28.1 vs 47.3.)
+TileOut tile_out(void* y, const void* bias = nullptr, int out_fp32 = 0) {
+  TileOut o{};
+  o.y = y;
+  o.bias = static_cast<const bf16_t*>(bias);
+  o.out_fp32 = out_fp32;
+  o.wide = (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+  return o;
+}
+
+// sid_linear takes the tile kernel from this many rows up, sid_linear_silu_mul from
+// kLinearSiluTiledMinM.
 constexpr int64_t kTiledMinM = 64;
-constexpr int64_t kTiledWideMinTiles = 512;
-// sid_linear_silu_mul takes the tiled form from this many rows up.
 constexpr int64_t kLinearSiluTiledMinM = 96;
 
 // K of the streaming kernel below, its chunk count and LDS row stride of staged x.
@@ -1407,20 +1580,6 @@ void launch_any(int nw, const void* x, int64_t ldx, const void* w, const void* b
 // The streaming kernel serves sid_linear from this many columns up (lm_head-sized N).
 constexpr int64_t kStreamMinN = 32768;
 
-// Persistent-grid size of the streaming kernel: one workgroup per CU of the current device.
-int stream_grid() {
-  static int count[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (count[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    count[dev] = n;
-  }
-  return count[dev];
-}
-
 // Row groups of up to 64 rows are streamed one after the other (the weights are re-read
 // per group); up to this many rows that still beats the tiled kernel on lm_head shapes.
 constexpr int64_t kStreamMaxM = 256;
@@ -1440,7 +1599,7 @@ void launch_stream_form(const bf16_t* x, int64_t ldx, const void* w, const void*
                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     attr_set = true;
   }
-  hipLaunchKernelGGL((linear_stream_kernel<MBS, AM, LEAN>), dim3(stream_grid()),
+  hipLaunchKernelGGL((linear_stream_kernel<MBS, AM, LEAN>), dim3(cu_count()),
                      dim3(STREAM_WAVES * 64), lds, s, x, ldx, (const bf16_t*)w,
                      (const bf16_t*)bias, y, m, n, out_fp32, bv, bi, cand_rows, row0);
 }
@@ -1600,18 +1759,8 @@ extern "C" int sid_linear(const void* x, int64_t ldx, const void* w, const void*
                          nullptr, nullptr, s);
     return check_launch("linear");
   }
-  if (m >= kTiledMinM || (m > MROWS && n >= kStreamMinN)) {
-    SID_REQUIRE((m + 63) / 64 <= 65535, "linear: too many rows");
-    const int64_t wide_tiles = ((m + 127) / 128) * ((n + 127) / 128);
-    if (wide_tiles >= kTiledWideMinTiles) {
-      launch_tiled<4, 2, 2, 4, 1>(x, ldx, w, bias, y, m, n, k, out_fp32, s);
-    } else if (((m + 127) / 128) * ((n + 63) / 64) <= stream_grid()) {
-      // At most one workgroup per CU: two sub-tiles in flight (measured, same bits: qkv
-      // M = 256 13.2 -> 11.2 us, o M = 2048 23.8 -> 18.6 us, down M = 2048 33.2 -> 24.9 us)
-      launch_tiled<4, 2, 2, 2, 2>(x, ldx, w, bias, y, m, n, k, out_fp32, s);
-    } else {
-      launch_tiled<4, 2, 2, 2, 1>(x, ldx, w, bias, y, m, n, k, out_fp32, s);
-    }
+  if (m >= kTiledMinM && tiles_fit(ldx, m, n, k)) {
+    launch_tiles<EPI_Y>(x, ldx, w, m, n, k, tile_out(y, bias, out_fp32), s);
     return check_launch("linear");
   }
   launch_any(pick_waves(n, m), x, ldx, w, bias, y, m, n, k, out_fp32, s);
@@ -1647,13 +1796,13 @@ extern "C" int sid_linear_partials(const void* x, int64_t ldx, const void* w, fl
 // one candidate per wave); more rows take the tiled GEMM with the argmax epilogue (one
 // candidate per 128-column tile, no logits needed: verify pass, 128 rows x 151936,
 // 101 us GEMM + 32 us argmax_rows before). Both reduce with argmax_finalize_kernel. The
-// workspace holds stream_grid() * STREAM_WAVES candidates per row, which bounds the tiled
+// workspace holds cu_count() * STREAM_WAVES candidates per row, which bounds the tiled
 // path's column tiles.
 static bool argmax_streams(int64_t m, int64_t n, int64_t k) {
   return m <= MROWS && stream_shape_ok(m, n, k);
 }
 
-static int64_t argmax_candidates() { return static_cast<int64_t>(stream_grid()) * STREAM_WAVES; }
+static int64_t argmax_candidates() { return static_cast<int64_t>(cu_count()) * STREAM_WAVES; }
 
 extern "C" int64_t sid_linear_argmax_workspace_bytes(int64_t m) {
   if (m < 1 || (m + MROWS - 1) / MROWS > 65535) return 0;
@@ -1688,7 +1837,11 @@ extern "C" int sid_linear_argmax(const void* x, int64_t ldx, const void* w, cons
     SID_REQUIRE(tiles <= cands, "linear_argmax: N=%lld has more than %lld column tiles",
                 (long long)n, (long long)cands);
     SID_REQUIRE((m + 127) / 128 <= 65535, "linear_argmax: too many rows");
-    launch_tiled<4, 2, 2, 4, 1, true>(x, ldx, w, bias, logits, m, n, k, 1, s, bv, bi);
+    SID_REQUIRE(tiles_fit(ldx, m, n, k), "linear_argmax: problem too large");
+    TileOut out = tile_out(logits, bias, 1);
+    out.best_val = bv;
+    out.best_idx = bi;
+    launch_tiles<EPI_ARGMAX>(x, ldx, w, m, n, k, out, s);
     used = static_cast<int>(tiles);
   }
   rc = check_launch("linear_argmax");
@@ -1700,7 +1853,7 @@ extern "C" int sid_linear_argmax(const void* x, int64_t ldx, const void* w, cons
 
 // Workspace of sid_linear_sample: 6 per-(wave, row) statistics + the finalize's lists.
 static int64_t sample_ws_bytes(int64_t m) {
-  const int64_t waves = static_cast<int64_t>(stream_grid()) * STREAM_WAVES;
+  const int64_t waves = static_cast<int64_t>(cu_count()) * STREAM_WAVES;
   return waves * m * 4 * 7;
 }
 
@@ -1724,7 +1877,7 @@ static void launch_sample_mbs(const bf16_t* x, int64_t ldx, const void* w, int m
                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     attr_set = true;
   }
-  hipLaunchKernelGGL((linear_sample_kernel<MBS>), dim3(stream_grid()), dim3(STREAM_WAVES * 64),
+  hipLaunchKernelGGL((linear_sample_kernel<MBS>), dim3(cu_count()), dim3(STREAM_WAVES * 64),
                      lds, s, x, ldx, (const bf16_t*)w, m, n, temps, seeds, pos, st, cand_rows,
                      row0);
 }
@@ -1762,7 +1915,7 @@ extern "C" int sid_linear_sample(const void* x, int64_t ldx, const void* w, int6
               "linear_sample: workspace must be 16-byte aligned");
   SID_REQUIRE(!(flags & 4) || logits == nullptr,
               "linear_sample: the streaming grouping writes no logits");
-  const int stream_groups = stream_grid() * STREAM_WAVES;
+  const int stream_groups = cu_count() * STREAM_WAVES;
   const int groups = tiled ? static_cast<int>((n + 127) / 128) : stream_groups;
   SID_REQUIRE(groups <= stream_groups, "linear_sample: N=%lld has more than %d column tiles",
               (long long)n, stream_groups);
@@ -1775,9 +1928,10 @@ extern "C" int sid_linear_sample(const void* x, int64_t ldx, const void* w, int6
   const int mi = static_cast<int>(m);
   if (tiled) {
     SID_REQUIRE((m + 127) / 128 <= 65535, "linear_sample: too many rows");
-    launch_tiled<4, 2, 2, 4, 1, false, false, true>(
-        x, ldx, w, nullptr, logits, m, n, k, 1, s, nullptr, nullptr,
-        SampleIn{temperatures, seeds, positions, st, m});
+    SID_REQUIRE(tiles_fit(ldx, m, n, k), "linear_sample: problem too large");
+    TileOut out = tile_out(logits, nullptr, 1);
+    out.sp = SampleIn{temperatures, seeds, positions, st, m};
+    launch_tiles<EPI_SAMPLE>(x, ldx, w, m, n, k, out, s);
     rc = check_launch("linear_sample");
     if (rc != SID_OK) return rc;
   } else {
@@ -1815,22 +1969,11 @@ extern "C" int sid_linear_silu_mul(const void* x, const void* w, void* out, int6
                   reinterpret_cast<uintptr_t>(out) % 4 == 0,
               "linear_silu_mul: misaligned operand");
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (m >= kLinearSiluTiledMinM && inter % 64 == 0) {
-    // From 96 rows: the tiled GEMM with the SwiGLU epilogue, in sid_linear's tile shapes
-    // (grid over the 2 * inter projection columns; the [M, 2 * inter] projection is never
-    // written). Same bits as the kernel below and as sid_linear + sid_silu_mul. Measured
-    // (I = 3072, weights from HBM, graph-timed): M = 64 11.9 us vs 9.8 for the kernel below,
-    // M = 96 12.4 vs 13.6, M = 128 12.8 vs 15.6, M = 192 12.5 vs 20.7; against sid_linear +
-    // sid_silu_mul M = 256 11.0 vs 15.1 us, M = 2048 38.4 vs 48.2, M = 8192 143 vs 171.
-    SID_REQUIRE((m + 127) / 128 <= 65535, "linear_silu_mul: too many rows");
-    const int64_t n = 2 * inter;
-    if (((m + 127) / 128) * ((n + 127) / 128) >= kTiledWideMinTiles) {
-      launch_tiled<4, 2, 2, 4, 1, false, true>(x, k, w, nullptr, out, m, n, k, 0, s);
-    } else if (((m + 127) / 128) * ((n + 63) / 64) <= stream_grid()) {
-      launch_tiled<4, 2, 2, 2, 2, false, true>(x, k, w, nullptr, out, m, n, k, 0, s);
-    } else {
-      launch_tiled<4, 2, 2, 2, 1, false, true>(x, k, w, nullptr, out, m, n, k, 0, s);
-    }
+  if (m >= kLinearSiluTiledMinM && inter % 64 == 0 && tiles_fit(k, m, 2 * inter, k)) {
+    // The tile kernel with the SwiGLU epilogue (grid over the 2 * inter projection columns;
+    // the [M, 2 * inter] projection is never written). Same bits as the kernel below and as
+    // sid_linear + sid_silu_mul.
+    launch_tiles<EPI_SWIGLU>(x, k, w, m, 2 * inter, k, tile_out(out), s);
     return check_launch("linear_silu_mul");
   }
   const int mbs = m >= MROWS ? 4 : static_cast<int>((m + 15) / 16);

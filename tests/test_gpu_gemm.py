@@ -166,3 +166,49 @@ def test_tiled_large_m_bitwise_matches_row_group_kernel(m, n, k):
     assert torch.equal(f32.to(torch.bfloat16), linear(x, w))
     ref = x[:64].float().cpu() @ w.float().cpu().t()
     torch.testing.assert_close(f32[:64].cpu(), ref, atol=3e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (64, 64, 256),       # one 64 x 64 tile, one chunk (the shortest K pipeline)
+    (300, 1024, 2048),   # 64 x 64 tiles, ragged rows
+    (1030, 1088, 768),   # 128 x 64 tiles, ragged rows
+    (1025, 3200, 256),   # 128 x 128 tiles, one row in the last ones, one chunk
+    (1500, 4032, 512),   # 256 x 128 tiles, half a tile of columns left
+    (4353, 8128, 256),   # 256 x 128 tiles, several rounds of the grid, one chunk
+])
+def test_tile_kernel_edges_bitwise(m, n, k):
+    """The pipelined tile GEMM in each tile shape, at the edges of tiles and of the K pipeline:
+    bits of the row-group kernel (row slices under 64 rows) for bf16 and fp32 outputs with and
+    without bias, from rows inside a wider matrix, into an output that is only 2- (4-) byte
+    aligned, with the rows after the output untouched; and the SwiGLU form against
+    sid_linear + sid_silu_mul."""
+    from sid.kernels.jit import load_ext
+    from sid.kernels.matmul_persistent import linear, linear_silu_mul
+    from sid.kernels.ops import silu_mul
+    ext = load_ext()
+    torch.manual_seed(m + n + k)
+    print(f"tile edges m={m} n={n} k={k}", flush=True)
+    big = torch.randn(m, k + 64, device="cuda", dtype=torch.bfloat16)
+    x = big[:, :k]
+    w = (torch.randn(n, k, device="cuda") * 0.05).to(torch.bfloat16)
+    b = torch.randn(n, device="cuda", dtype=torch.bfloat16)
+    rows = [(0, 48), (m - 33, m), (m // 2, m // 2 + 17)]
+    for bias in (None, b):
+        for fp32 in (False, True):
+            dt = torch.float32 if fp32 else torch.bfloat16
+            buf = torch.full((m * n + 9,), 7.0, device="cuda", dtype=dt)
+            for off in (0, 1):
+                y = buf[off:off + m * n].view(m, n)
+                ext.linear(x, w, bias, y, fp32)
+                for lo, hi in rows:
+                    assert torch.equal(y[lo:hi], linear(x[lo:hi].contiguous(), w, bias, fp32)), \
+                        (bias is not None, fp32, off, lo)
+                assert (buf[off + m * n:] == 7.0).all()
+    if k == 256:
+        return
+    x = x.contiguous()
+    if k != 1024:  # the SwiGLU entry takes K = 1024
+        x = torch.randn(m, 1024, device="cuda", dtype=torch.bfloat16)
+        w = (torch.randn(n, 1024, device="cuda") * 0.05).to(torch.bfloat16)
+    if (n // 2) % 64 == 0:
+        assert torch.equal(linear_silu_mul(x, w), silu_mul(linear(x, w)))
