@@ -37,6 +37,8 @@
 //                   before the PV product, as sid/kernels/extend_attention.py:106).
 #include "common.h"
 
+#include <type_traits>
+
 namespace sid {
 namespace {
 
@@ -82,12 +84,23 @@ __device__ __forceinline__ float pair32_sum(float v) {
 typedef short s16x4_v __attribute__((ext_vector_type(4)));
 typedef short s16x8_v __attribute__((ext_vector_type(8)));
 
+typedef __attribute__((address_space(3))) char* lds_char_t;
+
 // 4 bf16 of a V^T fragment through the LDS transpose read: within each 16-lane group,
 // lane L receives element L % 4 of the 8-byte values addressed by lanes L / 4 + 4j
 // (j = 0..3) of its group.
 __device__ __forceinline__ s16x4_v ld_tr16(const bf16_t* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
       (__attribute__((address_space(3))) s16x4_v*)(p));
+}
+
+// acc / l (l > 0), shared by every path that divides: y = 1 / l rounded, q = acc y, then one
+// correction (Markstein: the quotient correctly rounded), 5 operations for each of a row's
+// dims instead of a division's 12. An infinite or NaN q stays.
+__device__ __forceinline__ float div_row(float acc, float l, float y) {
+  const float q = acc * y;
+  const float c = __builtin_fmaf(__builtin_fmaf(-q, l, acc), y, q);
+  return __builtin_fabsf(q) < INFINITY ? c : q;
 }
 
 // Per-lane softmax state of one query row (the lane's 32 output dims).
@@ -127,6 +140,19 @@ __device__ __forceinline__ void fold(RowState& run, float m, float l, const f32x
 #pragma unroll
     for (int i = 0; i < 4; ++i) run.acc[db][i] = fold_elem(run.acc[db][i], a[db][i], f);
   run.m = f.mn;
+}
+
+// The row's output: acc / l rounded to bf16 (this lane: dims 16 db + 4 g .. +3).
+__device__ __forceinline__ void store_row(bf16_t* op, const RowState& run, int g) {
+  const float y = 1.0f / run.l;
+#pragma unroll
+  for (int db = 0; db < 8; ++db) {
+    const f32x4_v a = run.acc[db];
+    uint2 u;
+    u.x = pack_bf16x2(div_row(a[0], run.l, y), div_row(a[1], run.l, y));
+    u.y = pack_bf16x2(div_row(a[2], run.l, y), div_row(a[3], run.l, y));
+    *reinterpret_cast<uint2*>(op + 16 * db + 4 * g) = u;
+  }
 }
 
 struct Ctx {
@@ -232,6 +258,33 @@ __device__ __forceinline__ float softmax_tile(float (&s)[16], RowState& st, cons
   return rescale;
 }
 
+// p of a tile as the PV product's B operand (p is finite: exp of a finite difference, or 0).
+__device__ __forceinline__ void pack_p(bf16x8_v (&pf)[2], const float (&s)[16]) {
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb) {
+    uint4 u;
+    u.x = pack_bf16x2(s[8 * kb + 0], s[8 * kb + 1]);
+    u.y = pack_bf16x2(s[8 * kb + 2], s[8 * kb + 3]);
+    u.z = pack_bf16x2(s[8 * kb + 4], s[8 * kb + 5]);
+    u.w = pack_bf16x2(s[8 * kb + 6], s[8 * kb + 7]);
+    pf[kb] = __builtin_bit_cast(bf16x8_v, u);
+  }
+}
+
+// x * 1 == x: the rescale is skipped (same bits) unless some row of the wave moved its
+// reference maximum.
+__device__ __forceinline__ void apply_rescale(RowState& st, float rescale) {
+  if (__builtin_amdgcn_ballot_w64(rescale != 1.0f) != 0) {
+#pragma unroll
+    for (int db = 0; db < 8; ++db) {
+      st.acc[db][0] *= rescale;
+      st.acc[db][1] *= rescale;
+      st.acc[db][2] *= rescale;
+      st.acc[db][3] *= rescale;
+    }
+  }
+}
+
 // The 64-key tile starting at absolute key t0, already in LDS, folded into `st` (online
 // softmax).
 __device__ __forceinline__ void tile_math(RowState& st, const Ctx& c, int t0,
@@ -260,26 +313,8 @@ __device__ __forceinline__ void tile_math(RowState& st, const Ctx& c, int t0,
                                               : softmax_tile<true>(s, st, c, t0, sc2);
 
   bf16x8_v pf[2];
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    uint4 u;  // p is finite (exp of a finite difference, or 0)
-    u.x = pack_bf16x2(s[8 * kb + 0], s[8 * kb + 1]);
-    u.y = pack_bf16x2(s[8 * kb + 2], s[8 * kb + 3]);
-    u.z = pack_bf16x2(s[8 * kb + 4], s[8 * kb + 5]);
-    u.w = pack_bf16x2(s[8 * kb + 6], s[8 * kb + 7]);
-    pf[kb] = __builtin_bit_cast(bf16x8_v, u);
-  }
-  // x * 1 == x: the rescale is skipped (same bits) unless some row of the wave moved its
-  // reference maximum.
-  if (__builtin_amdgcn_ballot_w64(rescale != 1.0f) != 0) {
-#pragma unroll
-    for (int db = 0; db < 8; ++db) {
-      st.acc[db][0] *= rescale;
-      st.acc[db][1] *= rescale;
-      st.acc[db][2] *= rescale;
-      st.acc[db][3] *= rescale;
-    }
-  }
+  pack_p(pf, s);
+  apply_rescale(st, rescale);
 #pragma unroll
   for (int db = 0; db < 8; ++db) {
 #pragma unroll
@@ -320,13 +355,12 @@ __device__ __forceinline__ void run_tiles(RowState& st, const Ctx& c, int t_begi
 
 // part_* layout: [split][total_q][HQ]; part_a holds the unnormalised accumulator
 // (128 dims), part_ml = (m, l). Lane holds dims 16*db + 4*g .. +3 of its row.
-template <bool FANOUT>
-__global__ void __launch_bounds__(256) extend_attention_kernel(
+__global__ void __launch_bounds__(256) extend_fanout_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ qo_indptr,
     const int32_t* __restrict__ kv_indptr, const int32_t* __restrict__ kv_indices,
     int num_q_heads, int num_kv_heads, int64_t num_slots, float sm_scale, int mtiles,
-    int64_t total_q, bf16_t* __restrict__ o, float* __restrict__ part_a,
+    int64_t total_q, float* __restrict__ part_a,
     float* __restrict__ part_ml, int32_t* __restrict__ part_n) {
   __shared__ __align__(16) bf16_t sK[BN * KS_STRIDE];
   __shared__ __align__(16) bf16_t sV[BN * VS_STRIDE];
@@ -334,12 +368,8 @@ __global__ void __launch_bounds__(256) extend_attention_kernel(
 
   const int b = blockIdx.x;
   const int h_kv = blockIdx.y;
-  constexpr bool fanout = FANOUT;
-  // Without fan-out a workgroup walks every split up to its tile's causal limit, so late
-  // query tiles take longest: dispatch them first (blockIdx.z = 0 is the last tile).
-  const int mtile = fanout ? static_cast<int>(blockIdx.z) % mtiles
-                           : mtiles - 1 - static_cast<int>(blockIdx.z);
-  const int split = fanout ? static_cast<int>(blockIdx.z) / mtiles : 0;
+  const int mtile = static_cast<int>(blockIdx.z) % mtiles;
+  const int split = static_cast<int>(blockIdx.z) / mtiles;
 
   Ctx c;
   c.tid = threadIdx.x;
@@ -373,7 +403,7 @@ __global__ void __launch_bounds__(256) extend_attention_kernel(
   const int last_row = min(extend_len, (mtile + 1) * BQ) - 1;
   const int visible_end = min(kv_len, prefix + last_row + 1);
   const int nsplits = ceil_div(visible_end, KSPLIT);
-  if (fanout && split >= nsplits) return;  // the merge never reads this split
+  if (split >= nsplits) return;  // the merge never reads this split
 
   // q fragments (B operand of S^T = K Q^T): row qr, dims 32*ks + 8*g .. +7.
   bf16x8_v qf[4];
@@ -387,43 +417,211 @@ __global__ void __launch_bounds__(256) extend_attention_kernel(
   }
 
   const int64_t prow = static_cast<int64_t>(q_start + (c.row_ok ? qr : 0)) * num_q_heads + hq;
-  if constexpr (FANOUT) {
-    RowState st;
-    fresh(st);
-    run_tiles(st, c, split * KSPLIT, min(visible_end, (split + 1) * KSPLIT), qf, sc2, sK,
-              sV, s_idx);
-    if (!c.row_ok) return;
-    const int64_t pr = static_cast<int64_t>(split) * total_q * num_q_heads + prow;
-    float* pa = part_a + pr * D;
-#pragma unroll
-    for (int db = 0; db < 8; ++db)
-      *reinterpret_cast<f32x4_v*>(pa + 16 * db + 4 * c.g) = st.acc[db];
-    if (c.g == 0) {
-      part_ml[2 * pr] = st.m;
-      part_ml[2 * pr + 1] = st.l;
-      if (split == 0) part_n[prow] = nsplits;
-    }
-    return;
-  } else {
-  RowState run;
-  fresh(run);
-  for (int sp = 0; sp < nsplits; ++sp) {
-    RowState st;
-    fresh(st);
-    run_tiles(st, c, sp * KSPLIT, min(visible_end, (sp + 1) * KSPLIT), qf, sc2, sK, sV,
-              s_idx);
-    fold(run, st.m, st.l, st.acc);
-  }
+  RowState st;
+  fresh(st);
+  run_tiles(st, c, split * KSPLIT, min(visible_end, (split + 1) * KSPLIT), qf, sc2, sK,
+            sV, s_idx);
   if (!c.row_ok) return;
-  bf16_t* op = o + prow * D;
+  const int64_t pr = static_cast<int64_t>(split) * total_q * num_q_heads + prow;
+  float* pa = part_a + pr * D;
 #pragma unroll
-  for (int db = 0; db < 8; ++db) {
-    uint2 u;
-    u.x = pack_bf16x2(run.acc[db][0] / run.l, run.acc[db][1] / run.l);
-    u.y = pack_bf16x2(run.acc[db][2] / run.l, run.acc[db][3] / run.l);
-    *reinterpret_cast<uint2*>(op + 16 * db + 4 * c.g) = u;
+  for (int db = 0; db < 8; ++db)
+    *reinterpret_cast<f32x4_v*>(pa + 16 * db + 4 * c.g) = st.acc[db];
+  if (c.g == 0) {
+    part_ml[2 * pr] = st.m;
+    part_ml[2 * pr + 1] = st.l;
+    if (split == 0) part_n[prow] = nsplits;
   }
+}
+
+// ---- one workgroup per query tile: prefill, large decode-through-extend batches -----------
+//
+// Workgroup = (request, kv head, 8 NW query positions), NW waves; wave w: head w / (NW / 2),
+// one block of 16 query rows. The splits are walked in order with the tile math of the kernel
+// above (the same operations on the same values, so the same bits).
+//
+// What bounds it is instruction issue: a tile costs a wave 32 MFMAs (8 issue cycles each of
+// their 16) and 16 scores per lane through fma, exp, sum and pack, and everything else it
+// does per tile comes on top. So K and V are DMAed into two LDS buffers (no staging
+// registers, no LDS writes by the waves), the next tile in flight during a tile's math, with
+// one barrier per tile; the swizzled rows need no padding and little addressing; and a row's
+// 128 divisions share one reciprocal. 4 x 2048 tokens 162 -> 136 us (NW = 4) / 129 (NW = 8),
+// 1 x 2048 55 -> 50, 8420 ragged tokens 174 -> 154 / 138, 200 decode rows 168 -> 153.
+// Measured and not taken: softmax interleaved with the next tile's S MFMAs over four-deep
+// rings (141), two row blocks per wave (122, but 90 for 1 x 2048), six waves (173).
+//
+// LDS tiles are 64 rows of 256 bytes; 16-byte piece p of key's row sits at p ^ swz(key): over
+// the 16 keys of a fragment or transpose read swz takes 16 values.
+__device__ __forceinline__ int swz(int key) { return (key & 3) | (((key >> 3) & 3) << 2); }
+
+// Lane l's 16 bytes at its address -> LDS byte lds + 16 l.
+__device__ __forceinline__ void dma16(const void* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds)
+               : "memory");
+}
+__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off),
+               "s"(base), "s"(lds)
+               : "memory");
+}
+
+constexpr int kTileBytes = BN * D * 2;  // one K or V tile
+
+// OFF32: the pool is smaller than 4 GiB, so 32-bit offsets address it.
+template <int NW, bool OFF32>
+__global__ void __launch_bounds__(NW * 64, NW / 2) extend_prefill_kernel(
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
+    const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ qo_indptr,
+    const int32_t* __restrict__ kv_indptr, const int32_t* __restrict__ kv_indices,
+    int num_q_heads, int num_kv_heads, int64_t num_slots, float sm_scale, int mtiles,
+    bf16_t* __restrict__ o) {
+  extern __shared__ __align__(1024) char lds[];  // [2][K tile, V tile]
+  constexpr int ROWS = 8 * NW;  // query positions of the workgroup
+  const int b = blockIdx.x;
+  const int h_kv = blockIdx.y;
+  // Late query tiles walk the most keys: dispatch them first.
+  const int mtile = mtiles - 1 - static_cast<int>(blockIdx.z);
+  const int q_start = qo_indptr[b];
+  const int extend_len = qo_indptr[b + 1] - q_start;
+  if (mtile * ROWS >= extend_len) return;
+  const int kv_start = kv_indptr[b];
+  const int kv_len = kv_indptr[b + 1] - kv_start;
+  const int prefix = kv_len - extend_len;
+  if (prefix < 0) return;  // malformed batch: the kv range must cover the extend tokens
+
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int hq = h_kv * 2 + wave / (NW / 2);
+  const int w_row = mtile * ROWS + 16 * (wave % (NW / 2));  // the wave's first query row
+  const int qr = w_row + (lane & 15);
+  const bool row_ok = qr < extend_len;
+  const int64_t prow = static_cast<int64_t>(q_start + (row_ok ? qr : 0)) * num_q_heads + hq;
+  bf16x8_v qf[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    qf[ks] = *reinterpret_cast<const bf16x8_v*>(q + prow * D + 32 * ks + 8 * (lane >> 4));
+    if (!row_ok) qf[ks] = bf16x8_v{};
   }
+  const float sc2 = sm_scale * LOG2E;
+  const int last_row = min(extend_len, (mtile + 1) * ROWS) - 1;
+  const int ntiles = ceil_div(min(kv_len, prefix + last_row + 1), BN);
+  const int w_first = prefix + w_row;  // the wave's first and last positions
+  const int w_last = prefix + min(extend_len, w_row + 16) - 1;
+
+  // A wave loads KP pieces (4 keys, 1 KB) of the K tile and of the V tile, lane l key l / 16 of
+  // the piece; K and V rows share their offsets. A tile's slots are read one tile ahead.
+  constexpr int KP = 16 / NW;
+  const int32_t* idx = kv_indices + kv_start;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_char_t)lds));
+  const uint32_t max_slots = static_cast<uint32_t>(min<int64_t>(num_slots, 0x7fffffff));
+  const int row_bytes = num_kv_heads * D * 2;
+  const char* kbase = reinterpret_cast<const char*>(k_cache + h_kv * D);
+  const char* vbase = reinterpret_cast<const char*>(v_cache + h_kv * D);
+  struct Slots {
+    uint32_t s[KP];
+  };
+  auto load_slots = [&](int tile) {
+    Slots v;
+    const int key0 = tile * BN + 4 * wave + (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < KP; ++i) {
+      const int key = key0 + 4 * NW * i;
+      v.s[i] = key < kv_len ? idx[key] : 0;
+    }
+    return v;
+  };
+  auto load_tile_dma = [&](const Slots& v, int buf) {
+    int l = lane;  // opaque: per-lane constants are not kept in registers between tiles
+    asm volatile("" : "+v"(l));
+#pragma unroll
+    for (int i = 0; i < KP; ++i) {
+      const int key = 4 * (wave + NW * i) + (l >> 4);
+      const uint32_t slot = v.s[i] < max_slots ? v.s[i] : 0u;
+      const uint32_t piece = 16 * ((l & 15) ^ swz(key));
+      const uint32_t dst = lds0 + buf * 2 * kTileBytes + 1024u * (wave + NW * i);
+      if constexpr (OFF32) {  // fewer than 2^24 slots: rows are at least 256 bytes
+        const uint32_t off = __umul24(slot, row_bytes) + piece;
+        dma16(kbase, off, dst);
+        dma16(vbase, off, dst + kTileBytes);
+      } else {
+        const int64_t off = static_cast<int64_t>(slot) * row_bytes + piece;
+        dma16(kbase + off, dst);
+        dma16(vbase + off, dst + kTileBytes);
+      }
+    }
+  };
+
+  RowState run, st;
+  fresh(run);
+  fresh(st);
+  // One tile's math out of LDS buffer `buf`. MASK: some key is hidden from some row.
+  auto tile = [&](auto mask, int t0, int buf) {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    const int r = l & 15, g = l >> 4;
+    const int key_a0 = 8 * (r >> 2) + (r & 3);
+    const uint32_t ka = lds0 + buf * 2 * kTileBytes + key_a0 * 256 + 16 * (g ^ swz(key_a0));
+    f32x4_v s4[4];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {  // key block j, k-step ks
+      const int j = i & 3, ks = i >> 2;
+      const bf16x8_v kf = *(__attribute__((address_space(3))) const bf16x8_v*)(
+          (ka ^ (64u * ks)) + 256 * (32 * (j >> 1) + 4 * (j & 1)));
+      s4[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          kf, qf[ks], ks == 0 ? f32x4_v{0.0f, 0.0f, 0.0f, 0.0f} : s4[j], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    Ctx c;
+    c.g = g;
+    c.q_abs = w_first + r;
+    c.row_ok = row_ok;
+    float s[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = s4[i >> 2][i & 3];
+    const float rescale = softmax_tile<decltype(mask)::value>(s, st, c, t0, sc2);
+    bf16x8_v pf[2];
+    pack_p(pf, s);
+    __builtin_amdgcn_sched_barrier(0);
+    apply_rescale(st, rescale);
+    const int key_v = 8 * g + (r >> 2);
+    const uint32_t va = lds0 + (buf * 2 + 1) * kTileBytes + key_v * 256 +
+                        16 * (((r & 3) >> 1) ^ swz(key_v)) + 8 * (r & 1);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {  // dim block db, key half kb
+      const int db = i & 7, kb = i >> 3;
+      typedef __attribute__((address_space(3))) s16x4_v* tr_ptr_t;
+      const uint32_t p = (va ^ (32u * db)) + 8192 * kb;
+      const s16x4_v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)p);
+      const s16x4_v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr_t)(p + 1024));
+      const bf16x8_v vf = __builtin_bit_cast(
+          bf16x8_v, static_cast<s16x8_v>(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)));
+      st.acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[kb], st.acc[db], 0, 0, 0);
+    }
+  };
+
+  load_tile_dma(load_slots(0), 0);
+  Slots slots = load_slots(1);
+  for (int t = 0; t < ntiles; ++t) {
+    // Tile t has landed and every wave is done with the other buffer.
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if (t + 1 < ntiles) {
+      load_tile_dma(slots, (t + 1) & 1);
+      slots = load_slots(t + 2);
+    }
+    const int t0 = t * BN;
+    if (t0 + BN - 1 <= w_first && w_row < extend_len) {
+      tile(std::false_type{}, t0, t & 1);
+    } else if (t0 <= w_last && w_row < extend_len) {
+      tile(std::true_type{}, t0, t & 1);
+    }
+    if ((t & 3) == 3 || t + 1 == ntiles) {  // the split's end
+      fold(run, st.m, st.l, st.acc);
+      fresh(st);
+    }
+  }
+  if (row_ok) store_row(o + prow * D, run, lane >> 4);
 }
 
 // Fold the fanned-out split states of every (query row, head) item in split order: one
@@ -472,11 +670,14 @@ __global__ void __launch_bounds__(256) extend_merge_kernel(
       }
     }
   }
-  reinterpret_cast<uint32_t*>(o + item * D)[lane] = pack_bf16x2(acc.x / l, acc.y / l);
+  const float y = 1.0f / l;
+  reinterpret_cast<uint32_t*>(o + item * D)[lane] = pack_bf16x2(div_row(acc.x, l, y), div_row(acc.y, l, y));
 }
 
 // Fan the splits out when the grid would leave most CUs idle.
 constexpr int kFanoutBelowWg = 512;
+// 64-row workgroups in the grid from which they are used (4 per CU of 256).
+constexpr int64_t kWideWg = 1024;
 
 }  // namespace
 }  // namespace sid
@@ -524,11 +725,10 @@ extern "C" int sid_extend_attention_fwd(const void* q, const void* k_cache, cons
     float* pa = static_cast<float*>(workspace);
     float* pml = pa + static_cast<int64_t>(splits) * items * D;
     int32_t* pn = reinterpret_cast<int32_t*>(pml + static_cast<int64_t>(splits) * items * 2);
-    hipLaunchKernelGGL(extend_attention_kernel<true>, dim3(batch, num_kv_heads, mtiles * splits),
+    hipLaunchKernelGGL(extend_fanout_kernel, dim3(batch, num_kv_heads, mtiles * splits),
                        dim3(256), 0, s, (const bf16_t*)q, (const bf16_t*)k_cache,
                        (const bf16_t*)v_cache, qo_indptr, kv_indptr, kv_indices, num_q_heads,
-                       num_kv_heads, num_slots, sm_scale, mtiles, total_q, (bf16_t*)o, pa, pml,
-                       pn);
+                       num_kv_heads, num_slots, sm_scale, mtiles, total_q, pa, pml, pn);
     int rc = check_launch("extend_attention");
     if (rc != SID_OK) return rc;
     const int64_t groups = (items + 3) / 4;
@@ -538,9 +738,24 @@ extern "C" int sid_extend_attention_fwd(const void* q, const void* k_cache, cons
     return check_launch("extend_attention merge");
   }
   SID_REQUIRE(mtiles <= 65535, "extend_attention: grid too large");
-  hipLaunchKernelGGL(extend_attention_kernel<false>, dim3(batch, num_kv_heads, mtiles), dim3(256), 0, s,
-                     (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, qo_indptr,
-                     kv_indptr, kv_indices, num_q_heads, num_kv_heads, num_slots, sm_scale, mtiles,
-                     total_q, (bf16_t*)o, nullptr, nullptr, nullptr);
+  // 64-row workgroups (8 waves) load each key tile half as often, but a causal grid ends on
+  // its longest ones: from 4 of them per CU and 512 rows they win (4 x 2048 129 vs 136 us,
+  // 8420 ragged tokens 138 vs 154), below that the 32-row ones (1 x 4096 136 vs 148, 1 x 2048
+  // 50 vs 70, 200 x 1 over 1000 keys 153 vs 191).
+  auto prefill = [&](auto kern, int nw) {
+    const int mt = ceil_div(max_extend_len, 8 * nw);
+    hipLaunchKernelGGL(kern, dim3(batch, num_kv_heads, mt), dim3(nw * 64), 4 * kTileBytes, s,
+                       (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, qo_indptr,
+                       kv_indptr, kv_indices, num_q_heads, num_kv_heads, num_slots, sm_scale, mt,
+                       (bf16_t*)o);
+  };
+  const bool off32 = num_slots * num_kv_heads * D * 2 < (1ll << 32);
+  const bool wide = max_extend_len >= 512 && static_cast<int64_t>(batch) * num_kv_heads *
+                                                     ceil_div(max_extend_len, 64) >= kWideWg;
+  if (wide) {
+    off32 ? prefill(extend_prefill_kernel<8, true>, 8) : prefill(extend_prefill_kernel<8, false>, 8);
+  } else {
+    off32 ? prefill(extend_prefill_kernel<4, true>, 4) : prefill(extend_prefill_kernel<4, false>, 4);
+  }
   return check_launch("extend_attention");
 }

@@ -140,3 +140,46 @@ def test_split_fanout_bitwise_equals_sequential_fold(specs):
     c = torch.empty_like(q)
     ext.extend_attention_fwd(q, kb, vb, qo, kvp, idx, max_e, SCALE, c, 4 * max_kv, ws2)
     assert torch.equal(a, c)
+
+
+@pytest.mark.parametrize("specs,slots", [
+    # 32-row workgroups: one-row requests, tails of 32 rows and 64-key tiles, empty requests
+    ([(i % 5, 1 + (37 * i) % 70) for i in range(80)] + [(300, 0)], None),
+    # 64-row workgroups (512 rows and more, at least 1024 of them): ragged around tile edges
+    ([(0, 1024), (3, 1023), (0, 961), (17, 960), (0, 512), (255, 65), (0, 64), (1, 1)] +
+     [(0, 577 + i) for i in range(4)], None),
+    # a pool of more than 4 GiB a side (64-bit row offsets)
+    ([(0, 700), (40, 900)] + [(0, 33)] * 20, 2_200_000),
+], ids=["narrow", "wide", "big-pool"])
+def test_prefill_kernel_edges_bitwise(specs, slots):
+    """The one-workgroup-per-query-tile kernel against the split fan-out: every request's rows,
+    recomputed alone through the fan-out (grids below 512 workgroups take it), have the
+    same bits, also with out-of-range slots (they read slot 0) and an infinite V row."""
+    print(f"prefill edges {len(specs)} requests", flush=True)
+    q, kb, vb, qo, kvp, idx = _make(specs, seed=len(specs))
+    if slots is not None:  # spread the rows over a large pool, the last slot included
+        n = kb.shape[0]
+        at = torch.linspace(0, slots - 1, n, device="cuda", dtype=torch.float64).long()
+        big_k = torch.zeros(slots, HKV, D, device="cuda", dtype=torch.bfloat16)
+        big_v = torch.zeros_like(big_k)
+        big_k[at], big_v[at] = kb, vb
+        kb, vb, idx = big_k, big_v, at[idx.long()].int()
+    first = int(kvp[0])
+    hidden = int(kvp[1]) - 1  # the first request's last position
+    vb[idx[hidden].long(), :, 3] = float("inf")
+    idx[int(kvp[1])] = kb.shape[0]  # out of range: slot 0
+    idx[int(kvp[1]) + 1] = -1
+    assert first == 0
+    longest = max(e for _, e in specs)
+    tiles = -(-longest // 32)
+    assert len(specs) * HKV * tiles >= 512  # the full batch does not fan out
+    full = _fwd(q, kb, vb, qo, kvp, idx, longest, SCALE)
+    assert torch.isinf(full[int(qo[1]) - 1, :, 3]).all()  # (infinite, not NaN: inf / l)
+    for b in range(len(specs)):
+        lo, hi = int(qo[b]), int(qo[b + 1])
+        if hi == lo or (b > 12 and b % 9):
+            continue
+        one = _fwd(q[lo:hi].contiguous(), kb, vb, torch.tensor([0, hi - lo], dtype=torch.int32, device="cuda"),
+                   kvp[b:b + 2] - kvp[b], idx[int(kvp[b]):int(kvp[b + 1])].contiguous(), hi - lo, SCALE)
+        assert torch.equal(torch.nan_to_num(one), torch.nan_to_num(full[lo:hi])), (b, specs[b])
+        assert torch.equal(torch.isnan(one), torch.isnan(full[lo:hi])), b
