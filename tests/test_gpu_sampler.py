@@ -126,3 +126,46 @@ def test_positions_draws_equal_oracle_and_respect_top_p():
     got = _sample(logits, *args)
     assert torch.equal(got, sample_exact_ref(logits, *args))
     assert set(got.tolist()) <= {0, 1}
+
+
+@pytest.mark.parametrize("vocab", [151936, 20001, 1023, 7, 1])
+def test_list_and_full_paths_vs_exact_oracle(vocab):
+    """Rows whose cut lies in the listed columns (near the maximum), at the list's capacity
+    (8192 columns) and its threshold, beyond it (flat rows, nuclei wider than the list), with
+    long runs of equal keys at the cut, and with masked (-inf) columns; an odd vocabulary
+    puts rows off 16-byte alignment, tiny ones leave most parts of a row empty."""
+    g = torch.Generator().manual_seed(vocab + 1)
+    n = lambda *s: torch.randn(*s, generator=g)
+    rows, cfg = [], []
+
+    def add(row, t, k, p):
+        rows.append(row.to(torch.bfloat16).float())
+        cfg.append((t, k, p))
+
+    peaked = n(vocab) * 2.0
+    peaked[torch.randint(0, vocab, (min(40, vocab),), generator=g)] += 11.0
+    for t, k, p in ((0.6, 20, 0.95), (1.0, -1, 0.9), (0.7, 50, 1.0), (0.0, 5, 0.5), (1.0, -1, 1.0)):
+        add(peaked, t, k, p)
+    flat = n(vocab) * 0.3
+    for t, k, p in ((1.0, -1, 0.9), (1.0, 40, 1.0), (2.0, 3, 0.2), (1.0, -1, 0.0)):
+        add(flat, t, k, p)
+    for near in (8191, 8192, 8193):  # columns within the list's threshold, the rest far below
+        row = torch.full((vocab,), -40.0)
+        row[torch.randperm(vocab, generator=g)[:near]] = 0.0
+        row[vocab // 2] = 1.0
+        add(row, 1.0, 500, 1.0)
+        add(row, 1.0, -1, 0.5)
+        add(row, 1.0, 9000, 1.0)  # reaches past the list
+    edge = torch.full((vocab,), -9.703125)  # exp(-9.703125) just above 2^-14
+    edge[0] = 0.0
+    add(edge, 1.0, 10, 1.0)
+    add(edge - 0.0625 * torch.arange(vocab).clamp(max=3), 1.0, 3, 1.0)
+    masked = n(vocab) * 3.0
+    masked[torch.randperm(vocab, generator=g)[:vocab * 9 // 10]] = -math.inf
+    masked[vocab // 3] = 4.0
+    add(masked, 0.8, 30, 0.9)
+    add(masked, 0.8, vocab - 1, 1.0)
+    m = len(rows)
+    print(f"vocab={vocab} rows={m}", flush=True)
+    t, k, p = (list(x) for x in zip(*cfg))
+    _check(torch.stack(rows), t, k, p, [17 * i + 5 for i in range(m)], [31 * i for i in range(m)])
