@@ -71,10 +71,15 @@ def _check(cond: bool, msg: str) -> None:
 
 
 def _gpu(t: torch.Tensor, name: str, dtype: torch.dtype | None = None) -> None:
-    _check(isinstance(t, torch.Tensor) and t.is_cuda, f"{name} must be a GPU tensor")
-    _check(t.is_contiguous(), f"{name} must be contiguous")
-    if dtype is not None:
-        _check(t.dtype == dtype, f"{name} must be {dtype}, got {t.dtype}")
+    # The messages are built only when they are raised: formatting them (a dtype's repr above
+    # all) took half of an eager decode-attention call's host time (cache write + attention
+    # of one request, two calls with 13 tensors: 31 us for 12 us of kernels).
+    if not (isinstance(t, torch.Tensor) and t.is_cuda):
+        raise RuntimeError(f"{name} must be a GPU tensor")
+    if not t.is_contiguous():
+        raise RuntimeError(f"{name} must be contiguous")
+    if dtype is not None and t.dtype != dtype:
+        raise RuntimeError(f"{name} must be {dtype}, got {t.dtype}")
 
 
 def _ptr(t) -> int:
@@ -83,7 +88,8 @@ def _ptr(t) -> int:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """torch's current stream of the tensor's device (the raw handle: no Stream object)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 class NativeLib:
@@ -132,12 +138,15 @@ class NativeLib:
         flagged ORDER_EMPTY hold no tokens)."""
         _gpu(q, "q", torch.bfloat16)
         _check(q.dim() == 3, "q must be [B, HQ, D]")
-        b, hq, d = q.shape
-        for name, t in (("k_cache", k_cache), ("v_cache", v_cache)):
-            _gpu(t, name, torch.bfloat16)
-            _check(t.dim() == 3 and t.shape[2] == d, f"{name} must be [slots, HKV, {d}]")
-        _check(k_cache.shape == v_cache.shape, "k_cache and v_cache shapes differ")
-        hkv = k_cache.shape[1]
+        b, hq, d = qs = q.shape  # (each .shape builds a new object: taken once)
+        _gpu(k_cache, "k_cache", torch.bfloat16)
+        _gpu(v_cache, "v_cache", torch.bfloat16)
+        ks, vs = k_cache.shape, v_cache.shape
+        for name, sh in (("k_cache", ks), ("v_cache", vs)):
+            if not (len(sh) == 3 and sh[2] == d):
+                raise RuntimeError(f"{name} must be [slots, HKV, {d}]")
+        _check(ks == vs, "k_cache and v_cache shapes differ")
+        num_slots, hkv, _ = ks
         _gpu(kv_indptr, "kv_indptr", torch.int32)
         _check(kv_indptr.numel() == b + 1, "kv_indptr must have B+1 entries")
         _gpu(kv_indices, "kv_indices", torch.int32)
@@ -146,22 +155,22 @@ class NativeLib:
             _check(num_splits.numel() == b, "num_splits must have B entries")
         _gpu(part_o, "part_o", torch.float32)
         _gpu(part_lse, "part_lse", torch.float32)
-        _check(part_o.dim() == 4 and part_o.shape[1] == hq and part_o.shape[3] == d,
+        po, pl = part_o.shape, part_lse.shape
+        _check(len(po) == 4 and po[1] == hq and po[3] == d,
                "part_o workspace too small / wrong shape")
-        _check(part_lse.dim() == 3 and part_lse.shape[1] == hq
-               and part_lse.shape[2] == part_o.shape[2] and part_lse.shape[0] >= part_o.shape[0],
+        _check(len(pl) == 3 and pl[1] == hq and pl[2] == po[2] and pl[0] >= po[0],
                "part_lse workspace shape mismatch")
         _gpu(o, "o", torch.bfloat16)
-        _check(o.shape == q.shape, "o must have q's shape")
+        _check(o.shape == qs, "o must have q's shape")
         slots = int(max_splits) if grid_slots is None else int(grid_slots)
         order = self._order_ptr(wg_order, b * slots)
         _check(workers == 0 or wg_order is not None, "a worker launch needs wg_order")
         self._call("sid_flash_decode_workers_fwd", q.data_ptr(), k_cache.data_ptr(),
                    v_cache.data_ptr(), kv_indptr.data_ptr(), kv_indices.data_ptr(),
-                   _ptr(num_splits), b, hq, hkv, d, k_cache.shape[0], int(max_splits),
+                   _ptr(num_splits), b, hq, hkv, d, num_slots, int(max_splits),
                    int(fixed_split_size), int(segment_size), slots, int(variant), order,
                    float(sm_scale),
-                   part_o.data_ptr(), part_lse.data_ptr(), part_o.shape[0], part_o.shape[2],
+                   part_o.data_ptr(), part_lse.data_ptr(), po[0], po[2],
                    o.data_ptr(), int(workers), _stream(q))
 
     def flash_decode_fwd_noalloc(self, q, k_cache, v_cache, kv_indptr, kv_indices, num_splits,
@@ -175,7 +184,8 @@ class NativeLib:
         b, hq, d = q.shape
         for name, t in (("k_cache", k_cache), ("v_cache", v_cache)):
             _gpu(t, name, torch.bfloat16)
-            _check(t.dim() == 3 and t.shape[2] == d, f"{name} must be [slots, HKV, {d}]")
+            if not (t.dim() == 3 and t.shape[2] == d):
+                raise RuntimeError(f"{name} must be [slots, HKV, {d}]")
         _check(k_cache.shape == v_cache.shape, "k_cache and v_cache shapes differ")
         _gpu(kv_indptr, "kv_indptr", torch.int32)
         _check(kv_indptr.numel() == b + 1, "kv_indptr must have B+1 entries")
@@ -204,19 +214,19 @@ class NativeLib:
     def reshape_and_cache(self, k, v, k_cache, v_cache, slot_mapping) -> None:
         _gpu(k, "k", torch.bfloat16)
         _gpu(v, "v", torch.bfloat16)
-        _check(v.shape == k.shape, "v must have k's shape")
+        ks, cs = k.shape, k_cache.shape
+        _check(v.shape == ks, "v must have k's shape")
         _gpu(k_cache, "k_cache", torch.bfloat16)
         _gpu(v_cache, "v_cache", torch.bfloat16)
-        _check(k_cache.shape == v_cache.shape and k_cache.dim() == 3, "bad cache shapes")
-        _check(k.dim() == 3 and k.shape[1:] == k_cache.shape[1:],
-               "k must be [T, HKV, D] matching the cache")
+        _check(cs == v_cache.shape and len(cs) == 3, "bad cache shapes")
+        _check(len(ks) == 3 and ks[1:] == cs[1:], "k must be [T, HKV, D] matching the cache")
         _gpu(slot_mapping, "slot_mapping", torch.int64)
-        _check(slot_mapping.numel() == k.shape[0], "slot_mapping must have T entries")
-        if k.shape[0] == 0:
+        _check(slot_mapping.numel() == ks[0], "slot_mapping must have T entries")
+        if ks[0] == 0:
             return
         self._call("sid_reshape_and_cache", k.data_ptr(), v.data_ptr(), k_cache.data_ptr(),
-                   v_cache.data_ptr(), slot_mapping.data_ptr(), k.shape[0], k_cache.shape[1],
-                   k_cache.shape[2], k_cache.shape[0], _stream(k))
+                   v_cache.data_ptr(), slot_mapping.data_ptr(), ks[0], cs[1], cs[2],
+                   cs[0], _stream(k))
 
     # ---- the rest of the decode path ----------------------------------------------------
 
@@ -518,7 +528,8 @@ class NativeLib:
                             ("seeds", seeds, torch.int64), ("positions", positions, torch.int64),
                             ("out", out, torch.int64)):
             _gpu(t, name, dt)
-            _check(t.numel() == r, f"{name} must have one entry per row")
+            if t.numel() != r:
+                raise RuntimeError(f"{name} must have one entry per row")
         if r == 0:
             return
         ws = torch.empty(int(self.lib.sid_sample_workspace_bytes(r, v)), dtype=torch.uint8,
