@@ -15,10 +15,10 @@
 //     256-wide chunk of 64 columns per 4-wave workgroup, x chunk staged in LDS, weights
 //     streamed straight into MFMA B operands; writes partials[c][m][n], which the consumer
 //     kernel folds in chunk order (norm_rope.hip). No cross-workgroup synchronisation.
-//   * linear_kernel: direct y for M < 64 in one row group, every chunk of a column tile
-//     in one workgroup with the next chunk's operands prefetched during the MFMAs;
-//   * linear_tiled_kernel: direct y for M >= 64 (prefill, and decode / verify rows past the
-//     split-K cuts), LDS-tiled 128 x 128 / 128 x 64; also gate_up with the SwiGLU epilogue;
+//   * linear_tile_kernel: direct y (prefill, and decode / verify rows past the split-K cuts),
+//     persistent tiles of four shapes; also gate_up with the SwiGLU epilogue and the lm_head
+//     of more than 64 rows with the argmax or sampler epilogue;
+//   * linear_kernel: direct y for row strides past the tile kernel's 32-bit offsets;
 //   * linear_stream_kernel: lm_head-shaped N (persistent grid, x staged once per CU), with
 //     an optional fused greedy argmax.
 #include "common.h"
@@ -101,7 +101,7 @@ __device__ __forceinline__ void chunk_mfma(f32x4_v (&acc)[4], const bf16x8_v (&w
 
 // Direct y = x w^T (+ bias) for one 64-row group and 16*NW columns: every chunk in order,
 // the next chunk's weights and x prefetched into registers during the current chunk's
-// MFMAs. NW waves share one staged x chunk.
+// MFMAs. NW waves share one staged x chunk. (Only for sizes that tiles_fit refuses.)
 template <int NW>
 __global__ void __launch_bounds__(NW * 64) linear_kernel(
     const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ w,
@@ -361,6 +361,10 @@ __device__ __forceinline__ void sstate_store(const SampleStats& st, int64_t o, c
   st.a1i[o] = a.i1;
 }
 
+inline SampleStats sample_stats_at(const SampleStats& st, int64_t row) {
+  return {st.mx + row, st.sm + row, st.a1v + row, st.a1x + row, st.a2v + row, st.a1i + row};
+}
+
 // Per-row inputs of a fused sampler epilogue; statistics go to st at [group][cand_rows].
 struct SampleIn {
   const float* temps;
@@ -370,7 +374,7 @@ struct SampleIn {
   int64_t cand_rows;
 };
 
-// ---- pipelined tile GEMM (64 rows and more: prefill, verify passes, wide heads) ------------
+// ---- pipelined tile GEMM (direct projections of any M, verify passes, wide heads) ----------
 //
 // Persistent workgroups of WM x WN waves; wave (wm, wn) owns MB x NB MFMA blocks
 // (16 MB x 16 NB outputs) of a TM x TN tile. K streams in 64-deep sub-tiles through a ring of
@@ -522,7 +526,9 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) linear_tile_kernel(
     tile_mn(ok ? tt : 0, tm, tn);
     const int m0 = tm * TM;
     a = raw_srd(x + static_cast<int64_t>(m0) * ldx,
-                ok ? static_cast<uint32_t>(min(TM, M - m0)) * static_cast<uint32_t>(2 * ldx) : 0u);
+                ok ? static_cast<uint32_t>(min(TM, M - m0) - 1) * static_cast<uint32_t>(2 * ldx) +
+                         2u * K
+                   : 0u);
     int n0 = tn * TN, rows = min(TN, N - n0);
     if constexpr (EPI == EPI_SWIGLU) {
       const int inter = N / 2;
@@ -817,8 +823,8 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) linear_tile_kernel(
         if constexpr (EPI == EPI_SAMPLE) {
           sstate_store(out.sp.st, static_cast<int64_t>(tn) * out.sp.cand_rows + row, a);
         } else {
-          out.best_val[static_cast<int64_t>(tn) * M + row] = a.v1;
-          out.best_idx[static_cast<int64_t>(tn) * M + row] = a.i1;
+          out.best_val[static_cast<int64_t>(tn) * out.sp.cand_rows + row] = a.v1;
+          out.best_idx[static_cast<int64_t>(tn) * out.sp.cand_rows + row] = a.i1;
         }
       }
     }
@@ -898,9 +904,9 @@ void launch_tiles(const void* x, int64_t ldx, const void* w, int64_t m, int64_t 
   }
 }
 
-// Sizes whose tile offsets fit the kernel's 32-bit buffer ranges and indices.
+// Sizes whose tile offsets fit the kernel's 32-bit buffer ranges and indices (256 rows of x).
 bool tiles_fit(int64_t ldx, int64_t m, int64_t n, int64_t k) {
-  return ldx < (1ll << 22) && k < (1ll << 22) && m < (1ll << 31) && n < (1ll << 30);
+  return ldx < (1ll << 23) && k < (1ll << 23) && m < (1ll << 31) && n < (1ll << 30);
 }
 
 TileOut tile_out(void* y, const void* bias = nullptr, int out_fp32 = 0) {
@@ -912,10 +918,36 @@ TileOut tile_out(void* y, const void* bias = nullptr, int out_fp32 = 0) {
   return o;
 }
 
-// sid_linear takes the tile kernel from this many rows up, sid_linear_silu_mul from
-// kLinearSiluTiledMinM.
-constexpr int64_t kTiledMinM = 64;
-constexpr int64_t kLinearSiluTiledMinM = 96;
+// sid_linear_silu_mul takes the tile kernel above this many rows. Up to two 16-row blocks the
+// streaming kernel's eight-column workgroups put more weight loads in flight (I = 3072,
+// weights from HBM, streaming vs tiles, us: 16 rows 5.6 vs 7.3, 32 rows 6.6 vs 7.4; 48 rows
+// 7.8 vs 7.6, 64 rows 8.9 vs 7.9, 95 rows 12.6 vs 7.5; I = 9728: 32 rows 14.5 vs 12.3,
+// 64 rows 20.1 vs 13.8).
+constexpr int64_t kLinearSiluStreamMaxM = 32;
+
+// The lm_head epilogues' launch: 128-row tiles in slices of as many rows as the 32-bit
+// buffer offsets hold (one slice but for row strides of 16M elements and more).
+template <int EPI>
+void launch_head_tiles(const void* x, int64_t ldx, const void* w, int64_t m, int64_t n, int64_t k,
+                       const TileOut& out, hipStream_t s) {
+  const int64_t step = ldx < (1ll << 24) ? m : std::max<int64_t>(1, 0xffffffffll / (2 * ldx));
+  for (int64_t r0 = 0; r0 < m; r0 += step) {
+    TileOut o = out;
+    if (o.y != nullptr) o.y = static_cast<float*>(o.y) + r0 * n;
+    if constexpr (EPI == EPI_ARGMAX) {
+      o.best_val += r0;
+      o.best_idx += r0;
+    } else {
+      SampleIn& p = o.sp;
+      p.temps += r0;
+      p.seeds += r0;
+      p.positions += r0;
+      p.st = sample_stats_at(p.st, r0);
+    }
+    launch_tiles<EPI>(static_cast<const bf16_t*>(x) + r0 * ldx, ldx, w, std::min(step, m - r0), n,
+                      k, o, s);
+  }
+}
 
 // K of the streaming kernel below, its chunk count and LDS row stride of staged x.
 constexpr int WIDE_K = 1024;
@@ -1552,31 +1584,6 @@ int check_shapes(const void* x, int64_t ldx, const void* w, int64_t m, int64_t n
   return SID_OK;
 }
 
-template <int NW>
-void launch_linear(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t m,
-                   int64_t n, int64_t k, int out_fp32, hipStream_t stream) {
-  const dim3 grid((unsigned)(n / (16 * NW)), 1u, (unsigned)((m + MROWS - 1) / MROWS));
-  hipLaunchKernelGGL((linear_kernel<NW>), grid, dim3(NW * 64), 0, stream, (const bf16_t*)x, ldx,
-                     (const bf16_t*)w, (const bf16_t*)bias, y, m, n, k, out_fp32);
-}
-
-// Waves per workgroup: more waves share one staged x chunk (less L2->LDS traffic per
-// weight byte) but leave fewer workgroups; wide direct GEMMs (lm_head, prefill) use 8.
-// (16 waves would cap the kernel at 128 VGPRs and spill.)
-int pick_waves(int64_t n, int64_t m) {
-  const int64_t groups = (m + MROWS - 1) / MROWS;
-  if (n % 128 == 0 && (n / 128) * groups >= 512) return 8;
-  return 4;
-}
-
-void launch_any(int nw, const void* x, int64_t ldx, const void* w, const void* bias, void* y,
-                int64_t m, int64_t n, int64_t k, int out_fp32, hipStream_t s) {
-  switch (nw) {
-    case 8: return launch_linear<8>(x, ldx, w, bias, y, m, n, k, out_fp32, s);
-    default: return launch_linear<4>(x, ldx, w, bias, y, m, n, k, out_fp32, s);
-  }
-}
-
 // The streaming kernel serves sid_linear from this many columns up (lm_head-sized N).
 constexpr int64_t kStreamMinN = 32768;
 
@@ -1751,19 +1758,22 @@ extern "C" int sid_linear(const void* x, int64_t ldx, const void* w, const void*
   int rc = check_shapes(x, ldx, w, m, n, k, "linear");
   if (rc != SID_OK) return rc;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  // The streaming kernel reads the weights once per 64-row group; past one group the tiled
-  // kernel (each weight row reused by 128 rows) is faster: M = 128 151936 x 1024 fp32
-  // logits 165 -> 101 us, M = 256 327 -> 179 us (identical bits).
+  // The streaming kernel reads the weights once per 64-row group; past one group the tile
+  // kernel is faster (M = 128, 151936 x 1024 fp32 logits 165 vs 101 us, identical bits), and
+  // below kStreamMinN columns at any M: its loads run up to four sub-tiles ahead where the
+  // row-group kernel waits for each chunk. Weights from HBM, row group vs tiles, us:
+  // 1 x 1024 x 2048 15.4 vs 7.9, 32 x 1024 x 3072 29.9 vs 10.8, 16 x 4096 x 1024 10.6 vs 6.7,
+  // 63 x 12288 x 4096 59.7 vs 24.2, 1 x 64 x 512 5.8 vs 3.5.
   if (m <= MROWS && stream_shape_ok(m, n, k) && n >= kStreamMinN) {
     launch_stream<false>(x, ldx, w, bias, y, static_cast<int>(m), static_cast<int>(n), out_fp32,
                          nullptr, nullptr, s);
-    return check_launch("linear");
-  }
-  if (m >= kTiledMinM && tiles_fit(ldx, m, n, k)) {
+  } else if (tiles_fit(ldx, m, n, k)) {
     launch_tiles<EPI_Y>(x, ldx, w, m, n, k, tile_out(y, bias, out_fp32), s);
-    return check_launch("linear");
+  } else {
+    const dim3 grid((unsigned)(n / 64), 1u, (unsigned)((m + MROWS - 1) / MROWS));
+    hipLaunchKernelGGL((linear_kernel<4>), grid, dim3(256), 0, s, (const bf16_t*)x, ldx,
+                       (const bf16_t*)w, (const bf16_t*)bias, y, m, n, k, out_fp32);
   }
-  launch_any(pick_waves(n, m), x, ldx, w, bias, y, m, n, k, out_fp32, s);
   return check_launch("linear");
 }
 
@@ -1837,11 +1847,12 @@ extern "C" int sid_linear_argmax(const void* x, int64_t ldx, const void* w, cons
     SID_REQUIRE(tiles <= cands, "linear_argmax: N=%lld has more than %lld column tiles",
                 (long long)n, (long long)cands);
     SID_REQUIRE((m + 127) / 128 <= 65535, "linear_argmax: too many rows");
-    SID_REQUIRE(tiles_fit(ldx, m, n, k), "linear_argmax: problem too large");
+    SID_REQUIRE(k < (1ll << 23), "linear_argmax: K too large");
     TileOut out = tile_out(logits, bias, 1);
     out.best_val = bv;
     out.best_idx = bi;
-    launch_tiles<EPI_ARGMAX>(x, ldx, w, m, n, k, out, s);
+    out.sp.cand_rows = m;
+    launch_head_tiles<EPI_ARGMAX>(x, ldx, w, m, n, k, out, s);
     used = static_cast<int>(tiles);
   }
   rc = check_launch("linear_argmax");
@@ -1928,10 +1939,9 @@ extern "C" int sid_linear_sample(const void* x, int64_t ldx, const void* w, int6
   const int mi = static_cast<int>(m);
   if (tiled) {
     SID_REQUIRE((m + 127) / 128 <= 65535, "linear_sample: too many rows");
-    SID_REQUIRE(tiles_fit(ldx, m, n, k), "linear_sample: problem too large");
     TileOut out = tile_out(logits, nullptr, 1);
     out.sp = SampleIn{temperatures, seeds, positions, st, m};
-    launch_tiles<EPI_SAMPLE>(x, ldx, w, m, n, k, out, s);
+    launch_head_tiles<EPI_SAMPLE>(x, ldx, w, m, n, k, out, s);
     rc = check_launch("linear_sample");
     if (rc != SID_OK) return rc;
   } else {
@@ -1969,7 +1979,7 @@ extern "C" int sid_linear_silu_mul(const void* x, const void* w, void* out, int6
                   reinterpret_cast<uintptr_t>(out) % 4 == 0,
               "linear_silu_mul: misaligned operand");
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (m >= kLinearSiluTiledMinM && inter % 64 == 0 && tiles_fit(k, m, 2 * inter, k)) {
+  if (m > kLinearSiluStreamMaxM && inter % 64 == 0 && tiles_fit(k, m, 2 * inter, k)) {
     // The tile kernel with the SwiGLU epilogue (grid over the 2 * inter projection columns;
     // the [M, 2 * inter] projection is never written). Same bits as the kernel below and as
     // sid_linear + sid_silu_mul.

@@ -28,14 +28,17 @@ from sid.kernels.rope import RotaryEmbedding
 
 
 # Split-K projections (chunk partials folded by the consuming fused kernel) or direct GEMMs
-# (the tiled kernel from 64 rows): both give identical bits, so this is a speed choice per
-# projection shape. With W = SPLIT_K_MAX_TOKENS: outputs of N <= 2048 columns (o, down: few
-# output tiles) split up to 3 W rows, N <= 4096 (qkv) below 5 W / 8, wider ones below W.
-# The native executor applies the same rule (sid_qwen3_model.split_k_max_tokens). MI355X,
-# weights from HBM, consumers included (split vs direct, us): o at 512 rows 18.9 vs 20.1,
-# at 1024 27.6 vs 23.4; down 21.8 vs 28.6, 36.8 vs 31.2; qkv at 128 rows 14.5 vs 15.8, at
-# 192 17.9 vs 15.8, at 256 20.7 vs 16.2.
-SPLIT_K_MAX_TOKENS = 256
+# (the tile kernel): both give identical bits, so this is a speed choice per projection
+# shape. With W = SPLIT_K_MAX_TOKENS: outputs of N <= 2048 columns (o, down: few output
+# tiles) split up to 3 W rows, N <= 4096 (qkv) below 5 W / 8, wider ones below W. The native
+# executor applies the same rule (sid_qwen3_model.split_k_max_tokens). MI355X, weights from
+# HBM, consumers included (split vs direct, us): o at 128 rows 8.9 vs 11.0, at 192 11.2 vs
+# 10.9, at 512 17.2 vs 11.7; down at 256 rows 15.9 vs 18.4, at 384 17.8 vs 18.7, at 512 20.4
+# vs 19.0, at 768 26.3 vs 19.1; qkv at 64 rows 9.2 vs 10.2, at 72 11.2 vs 9.7, at 128 13.2 vs
+# 10.5. Inside a whole prefill (28 layers, split vs direct o and down): 320 rows 2.11 vs 2.26
+# ms, 400 rows 2.32 vs 2.27, 512 rows 2.45 vs 2.42, 640 rows 2.90 vs 2.68, 750 rows 3.24 vs
+# 2.91, hence 3 W = 384.
+SPLIT_K_MAX_TOKENS = 128
 
 
 def split_k_preferred(rows: int, n: int, wide_max: int = SPLIT_K_MAX_TOKENS) -> bool:

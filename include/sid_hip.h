@@ -425,7 +425,7 @@ int sid_linear_argmax(const void* x, int64_t ldx, const void* w, const void* bia
  * Results are bit-identical to issuing the same entry points one by one. It
  * has no counterpart of its own in the reference, whose forward is Python.
  * A projection with N <= 2048 output columns uses the split-K path up to
- * 4 * split_k_max_tokens tokens, N <= 4096 up to split_k_max_tokens, wider ones
+ * 3 * split_k_max_tokens tokens, N <= 4096 below 5/8 of split_k_max_tokens, wider ones
  * below split_k_max_tokens (the results are the same either way). When the
  * layer's packed weights (sid_pack_decode_weight) are given and the batch has
  * at most chain_max_tokens tokens, each layer instead runs the decode-step

@@ -169,6 +169,9 @@ def test_tiled_large_m_bitwise_matches_row_group_kernel(m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [
+    (1, 64, 256),        # one row
+    (33, 128, 1024),     # one tile of rows, the first SwiGLU rows on tiles
+    (63, 1024, 3072),    # a row short of a tile
     (64, 64, 256),       # one 64 x 64 tile, one chunk (the shortest K pipeline)
     (300, 1024, 2048),   # 64 x 64 tiles, ragged rows
     (1030, 1088, 768),   # 128 x 64 tiles, ragged rows
@@ -178,7 +181,7 @@ def test_tiled_large_m_bitwise_matches_row_group_kernel(m, n, k):
 ])
 def test_tile_kernel_edges_bitwise(m, n, k):
     """The pipelined tile GEMM in each tile shape, at the edges of tiles and of the K pipeline:
-    bits of the row-group kernel (row slices under 64 rows) for bf16 and fp32 outputs with and
+    bits of the split-K kernel's chunks folded in order, for bf16 and fp32 outputs with and
     without bias, from rows inside a wider matrix, into an output that is only 2- (4-) byte
     aligned, with the rows after the output untouched; and the SwiGLU form against
     sid_linear + sid_silu_mul."""
@@ -192,17 +195,20 @@ def test_tile_kernel_edges_bitwise(m, n, k):
     x = big[:, :k]
     w = (torch.randn(n, k, device="cuda") * 0.05).to(torch.bfloat16)
     b = torch.randn(n, device="cuda", dtype=torch.bfloat16)
-    rows = [(0, 48), (m - 33, m), (m // 2, m // 2 + 17)]
+    part = torch.empty(k // 256, m, n, device="cuda", dtype=torch.float32)
+    ext.linear_partials(x, w, part)
+    fold = part[0].clone()
+    for c in range(1, k // 256):
+        fold += part[c]
     for bias in (None, b):
+        ref = (fold if bias is None else fold + b.float()).to(torch.bfloat16)
         for fp32 in (False, True):
             dt = torch.float32 if fp32 else torch.bfloat16
             buf = torch.full((m * n + 9,), 7.0, device="cuda", dtype=dt)
             for off in (0, 1):
                 y = buf[off:off + m * n].view(m, n)
                 ext.linear(x, w, bias, y, fp32)
-                for lo, hi in rows:
-                    assert torch.equal(y[lo:hi], linear(x[lo:hi].contiguous(), w, bias, fp32)), \
-                        (bias is not None, fp32, off, lo)
+                assert torch.equal(y, ref.to(dt)), (bias is not None, fp32, off)
                 assert (buf[off + m * n:] == 7.0).all()
     if k == 256:
         return
@@ -212,3 +218,28 @@ def test_tile_kernel_edges_bitwise(m, n, k):
         w = (torch.randn(n, 1024, device="cuda") * 0.05).to(torch.bfloat16)
     if (n // 2) % 64 == 0:
         assert torch.equal(linear_silu_mul(x, w), silu_mul(linear(x, w)))
+
+
+@pytest.mark.parametrize("m,ldx", [(2, 1 << 23), (65, 1 << 25)])
+def test_wide_row_strides(m, ldx):
+    """Rows further apart than 32-bit tile offsets reach (the last token of each of m long
+    sequences): the bits of the same rows packed, from sid_linear and the lm_head's argmax."""
+    from sid.kernels.jit import load_ext
+    from sid.kernels.matmul_persistent import linear
+    ext = load_ext()
+    print(f"wide row stride m={m} ldx={ldx}", flush=True)
+    n, k = 320, 512
+    packed = torch.randn(m, k, device="cuda", dtype=torch.bfloat16)
+    big = torch.empty(m, ldx, device="cuda", dtype=torch.bfloat16)
+    x = big[:, :k]
+    x.copy_(packed)
+    w = (torch.randn(n, k, device="cuda") * 0.05).to(torch.bfloat16)
+    ref = linear(packed, w, None, True)
+    y = torch.empty(m, n, device="cuda", dtype=torch.float32)
+    ext.linear(x, w, None, y, True)
+    assert torch.equal(y, ref)
+    logits = torch.empty_like(y)
+    out = torch.empty(m, device="cuda", dtype=torch.int64)
+    ws = torch.empty(ext.linear_argmax_workspace_bytes(m), device="cuda", dtype=torch.uint8)
+    ext.linear_argmax(x, w, None, logits, ws, out)
+    assert torch.equal(logits, ref) and torch.equal(out, ref.argmax(1))
