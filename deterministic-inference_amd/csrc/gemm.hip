@@ -964,8 +964,8 @@ constexpr int WXS = WIDE_K + 8;
 // chunk's MFMA sequence and the left fold of the four chunks are those of linear_kernel,
 // so the logits have the same bits. With ARGMAX, each lane keeps the best (value, column)
 // of the rows it holds over its wave's columns (the values compared are the bf16-rounded
-// logits the unfused path writes); the wave's best per row goes to a workspace
-// [waves][M] that argmax_finalize_kernel reduces. The (value, index) order is total
+// logits the unfused path writes); the workgroup's best per row goes to a workspace
+// [workgroups][M] that argmax_finalize_kernel reduces. The (value, index) order is total
 // (torch's: larger value, then smaller index; NaN above everything, first NaN wins), so
 // the result does not depend on how the columns are split.
 constexpr int STREAM_WAVES = 8;
@@ -1121,37 +1121,72 @@ __global__ void __launch_bounds__(STREAM_WAVES * 64) linear_stream_kernel(
             ix = oi;
           }
         }
-        const int row = 16 * mb + 4 * g + i;
-        if (r == 0 && row < M) {
-          best_val[static_cast<int64_t>(gw) * cand_rows + row0 + row] = v;
-          best_idx[static_cast<int64_t>(gw) * cand_rows + row0 + row] = ix;
+        bv[mb][i] = v;
+        bi[mb][i] = ix;
+      }
+    }
+    // Then over the workgroup's waves (x is no longer read, its LDS is reused): one candidate
+    // per row and workgroup for the finalize to gather from lines that hold all rows (a
+    // candidate per wave: 64 rows x 2048 candidates took the finalize 7.3 us, 256 take 4.8;
+    // 64 x 151936 greedy 75.7 -> 71.9 us in all).
+    __syncthreads();
+    float* s_v = reinterpret_cast<float*>(lx);
+    int* s_i = reinterpret_cast<int*>(s_v + STREAM_WAVES * ROWS);
+    if (r == 0) {
+#pragma unroll
+      for (int mb = 0; mb < MBS; ++mb) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          s_v[wave * ROWS + 16 * mb + 4 * g + i] = bv[mb][i];
+          s_i[wave * ROWS + 16 * mb + 4 * g + i] = bi[mb][i];
         }
       }
+    }
+    __syncthreads();
+    const int row = threadIdx.x;
+    if (row < M && row < ROWS) {
+      float v = s_v[row];
+      int ix = s_i[row];
+#pragma unroll
+      for (int q = 1; q < STREAM_WAVES; ++q) {
+        const float ov = s_v[q * ROWS + row];
+        const int oi = s_i[q * ROWS + row];
+        if (argmax_better(ov, oi, v, ix)) {
+          v = ov;
+          ix = oi;
+        }
+      }
+      best_val[static_cast<int64_t>(blockIdx.x) * cand_rows + row0 + row] = v;
+      best_idx[static_cast<int64_t>(blockIdx.x) * cand_rows + row0 + row] = ix;
     }
   }
 }
 
-// Per row: the best of the per-wave candidates (any order gives the same answer).
+// Per row: the best of the candidates (any order gives the same answer).
 __global__ void __launch_bounds__(256) argmax_finalize_kernel(const float* __restrict__ best_val,
                                                               const int* __restrict__ best_idx,
-                                                              int num_waves, int M,
+                                                              int num_cands, int M,
                                                               int64_t* __restrict__ out) {
   const int row = blockIdx.x;
   float v = -INFINITY;
   int ix = 0x7fffffff;
-  // Eight candidates per thread loaded at once (one round trip for the 2048 waves of the
-  // persistent grid instead of eight); the order is total, so the visiting order is free.
+  // Eight candidates per thread loaded at once (one round trip for up to 2048 of the tiled
+  // path instead of eight); the order is total, so the visiting order is free.
   constexpr int U = 8;
-  for (int base = threadIdx.x; base < num_waves; base += 256 * U) {
+  for (int base = threadIdx.x; base < num_cands; base += 256 * U) {
     float cv[U];
     int ci[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int wv = base + 256 * u;
-      const bool in = wv < num_waves;
-      const int64_t off = static_cast<int64_t>(in ? wv : 0) * M + row;
-      cv[u] = in ? best_val[off] : -INFINITY;
-      ci[u] = in ? best_idx[off] : 0x7fffffff;
+      const bool in = wv < num_cands;
+      const int64_t off = static_cast<int64_t>(wv) * M + row;
+      cv[u] = -INFINITY;
+      ci[u] = 0x7fffffff;
+      if (in) {
+        cv[u] = best_val[off];
+        ci[u] = best_idx[off];
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -1627,7 +1662,7 @@ void launch_stream_mbs(const bf16_t* x, int64_t ldx, const void* w, const void* 
 }
 
 // One launch per 64-row group; group g reads x rows 64g.., writes y rows 64g.. and the
-// candidate rows 64g.. of the [waves][m] workspace.
+// candidate rows 64g.. of the [workgroups][m] workspace.
 template <bool AM>
 void launch_stream(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int m,
                    int n, int out_fp32, float* bv, int* bi, hipStream_t s) {
@@ -1803,7 +1838,7 @@ extern "C" int sid_linear_partials(const void* x, int64_t ldx, const void* w, fl
 }
 
 // sid_linear_argmax: up to one 64-row group streams the weights once (linear_stream_kernel,
-// one candidate per wave); more rows take the tiled GEMM with the argmax epilogue (one
+// one candidate per workgroup); more rows take the tiled GEMM with the argmax epilogue (one
 // candidate per 128-column tile, no logits needed: verify pass, 128 rows x 151936,
 // 101 us GEMM + 32 us argmax_rows before). Both reduce with argmax_finalize_kernel. The
 // workspace holds cu_count() * STREAM_WAVES candidates per row, which bounds the tiled
@@ -1841,7 +1876,7 @@ extern "C" int sid_linear_argmax(const void* x, int64_t ldx, const void* w, cons
   if (argmax_streams(m, n, k)) {
     launch_stream<true>(x, ldx, w, bias, logits, static_cast<int>(m), static_cast<int>(n), 1, bv,
                         bi, s);
-    used = static_cast<int>(cands);
+    used = cu_count();
   } else {
     const int64_t tiles = (n + 127) / 128;
     SID_REQUIRE(tiles <= cands, "linear_argmax: N=%lld has more than %lld column tiles",
