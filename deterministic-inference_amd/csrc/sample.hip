@@ -44,8 +44,10 @@ __device__ __forceinline__ bool better(float v, int64_t i, float bv, int64_t bi)
 // the columns above a few thresholds, sample_list_kernel lists the columns above the first
 // threshold that should hold the cut. sample_select_kernel, one workgroup per row, finds the
 // cut and draws over the list in LDS: tens to thousands of keys instead of the vocabulary.
-// Rows whose cut is not provably among 16384 columns (flat distributions, non-finite sums),
-// or without limits, take the passes over all columns there. One 1024-thread workgroup per
+// Rows whose cut is not provably among 16384 columns (flat distributions, non-finite sums)
+// take the passes over all columns there; rows without limits draw in the third launch, part
+// by part (one 1024-thread workgroup per row vs now, us: 1 row 123 vs 40, 64 rows 132 vs 68,
+// 128 rows 137 vs 113; 256 rows, whose workgroups filled the chip, 151 vs 191). One 1024-thread workgroup per
 // row for everything, nine passes over 151936 columns bound by one CU's latency and LDS
 // atomics, took 205 us for 1 row and 366 for 64 (top-k / top-p mixes over peaked rows); these
 // four take 30 and 72 (max 6 / 11, sum 12 / 30, list 6 / 12, select 9 / 20). Listing in the
@@ -312,9 +314,29 @@ __device__ __forceinline__ float row_max(const PartStats& st, int64_t r, float t
   return mx / t;
 }
 
+__device__ __forceinline__ float row_sum(const PartStats& st, int64_t r) {
+  float sum = st.sum[r * kParts];
+  for (int q = 1; q < kParts; ++q) sum += st.sum[r * kParts + q];
+  return sum;
+}
+
+// A row's limits: ranks and fixed-point mass before a kept rank.
+struct Limits {
+  uint64_t k, mass;
+  bool truncate;
+};
+__device__ __forceinline__ Limits limits_of(int64_t k, float tp, int64_t cols) {
+  Limits l;
+  l.k = (k > 0 && k < cols) ? static_cast<uint64_t>(k) : static_cast<uint64_t>(cols);
+  l.mass = tp < 1.0f ? (tp > 0.0f ? static_cast<uint64_t>(static_cast<double>(tp) * kMassUnit) : 0ull)
+                     : ~0ull;
+  l.truncate = tp < 1.0f || l.k < static_cast<uint64_t>(cols);
+  return l;
+}
+
 __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
-    const float* __restrict__ logits, int64_t ld, const float* __restrict__ temps, int cols,
-    PartStats st) {
+    const float* __restrict__ logits, int64_t ld, const float* __restrict__ temps,
+    const int64_t* __restrict__ top_ks, const float* __restrict__ top_ps, int cols, PartStats st) {
   __shared__ __align__(16) float4 s_e[kPartSteps][64];
   __shared__ int s_count[kPartThreads / 64][kCuts];
   __shared__ float s_mass[kPartThreads / 64][kCuts];
@@ -324,6 +346,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
   const float* row = logits + r * ld;
   const float t = temps[r];
   if (!(t > 0.0f)) return;  // greedy row
+  const bool cuts = limits_of(top_ks[r], top_ps[r], cols).truncate;
   const PartCols pc = part_cols(row, cols, q);
   const float mx = row_max(st, r, t);
   const Quot div = quot_of(t);
@@ -331,7 +354,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
   float m_cut[kCuts] = {};
   auto exp_of = [&](float v, bool valid) {
     const float e = expf(quot(v, div) - mx);
-    const bool hit = valid && e >= kCutMin[kCuts - 1];
+    const bool hit = cuts && valid && e >= kCutMin[kCuts - 1];
     if (__builtin_amdgcn_ballot_w64(hit) != 0) {
 #pragma unroll
       for (int j = 0; j < kCuts; ++j) {
@@ -417,7 +440,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
     }
   }
   __syncthreads();
-  if (threadIdx.x < kCuts) {
+  if (cuts && threadIdx.x < kCuts) {
     int n = 0;
     float m = 0.0f;
     for (int w = 0; w < kPartThreads / 64; ++w) {
@@ -430,18 +453,83 @@ __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
   if (threadIdx.x == 0) st.sum[blockIdx.x] = part;
 }
 
-// A row's limits: ranks and fixed-point mass before a kept rank.
-struct Limits {
-  uint64_t k, mass;
-  bool truncate;
-};
-__device__ __forceinline__ Limits limits_of(int64_t k, float tp, int64_t cols) {
-  Limits l;
-  l.k = (k > 0 && k < cols) ? static_cast<uint64_t>(k) : static_cast<uint64_t>(cols);
-  l.mass = tp < 1.0f ? (tp > 0.0f ? static_cast<uint64_t>(static_cast<double>(tp) * kMassUnit) : 0ull)
-                     : ~0ull;
-  l.truncate = tp < 1.0f || l.k < static_cast<uint64_t>(cols);
-  return l;
+// A row without limits: the best draw over the part's columns. e / sum as quot: exact to the
+// bit wherever it reaches 2^-59, and below that p + 1e-10 is 1e-10 either way. (In the select,
+// one workgroup per row drew over all columns: 1 row 114 us in all, 256 rows 225.)
+__device__ __forceinline__ void draw_all(const float* __restrict__ row, int cols, int q, float t,
+                                         float mx, float sum, uint32_t row_hash, float* best,
+                                         int32_t* best_at) {
+  __shared__ float s_v[kPartThreads / 64];
+  __shared__ int s_i[kPartThreads / 64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const PartCols pc = part_cols(row, cols, q);
+  const Quot div = quot_of(t), inv = quot_of(sum);
+  float bv = -INFINITY;
+  int bi = 0x7fffffff;
+  auto take = [&](float v, int c) {
+    const float p = quot(expf(quot(v, div) - mx), inv);
+    const float s = logf(p + kSampleEps) + seeded_gumbel(row_hash, c);
+    if (better(s, c, bv, bi)) {
+      bv = s;
+      bi = c;
+    }
+  };
+  constexpr int U = kPartSteps / 4;
+  for (int m0 = 0; m0 < pc.steps; m0 += kPartSteps) {
+    float4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = 64 * q + lane + kSampleThreads * (m0 + wave + 4 * u);
+      v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (i < pc.vecs) {
+        if (pc.vec) {
+          v[u] = reinterpret_cast<const float4*>(row)[i];
+        } else {
+          v[u].x = row[i];
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = 64 * q + lane + kSampleThreads * (m0 + wave + 4 * u);
+      if (i < pc.vecs) {
+        if (pc.vec) {
+          take(v[u].x, 4 * i);
+          take(v[u].y, 4 * i + 1);
+          take(v[u].z, 4 * i + 2);
+          take(v[u].w, 4 * i + 3);
+        } else {
+          take(v[u].x, i);
+        }
+      }
+    }
+  }
+  if (pc.vec && q == 0 && wave == 0 && 4 * pc.vecs + lane < cols)
+    take(row[4 * pc.vecs + lane], 4 * pc.vecs + lane);
+  for (int mask = 1; mask < 64; mask <<= 1) {
+    const float ov = lane_xor(bv, mask);
+    const int oi = __builtin_amdgcn_ds_bpermute((lane ^ mask) << 2, bi);
+    if (better(ov, oi, bv, bi)) {
+      bv = ov;
+      bi = oi;
+    }
+  }
+  if (lane == 0) {
+    s_v[wave] = bv;
+    s_i[wave] = bi;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kPartThreads / 64; ++w) {
+      if (better(s_v[w], s_i[w], bv, bi)) {
+        bv = s_v[w];
+        bi = s_i[w];
+      }
+    }
+    *best = bv;
+    *best_at = bi;
+  }
 }
 
 // (bound: one read of the logits from L2 / the last-level cache and the launch; sum: also ~45
@@ -452,8 +540,9 @@ __device__ __forceinline__ Limits limits_of(int64_t k, float tp, int64_t cols) {
 // those take an exponential.
 __global__ void __launch_bounds__(kPartThreads) sample_list_kernel(
     const float* __restrict__ logits, int64_t ld, const float* __restrict__ temps,
-    const int64_t* __restrict__ top_ks, const float* __restrict__ top_ps, int cols, PartStats st,
-    uint32_t* __restrict__ lists) {
+    const int64_t* __restrict__ top_ks, const float* __restrict__ top_ps,
+    const int64_t* __restrict__ seeds, const int64_t* __restrict__ positions, int cols,
+    PartStats st, uint32_t* __restrict__ lists) {
   __shared__ int s_cnt[kCuts];
   __shared__ float s_mass[kCuts];
   __shared__ int s_n;
@@ -464,8 +553,12 @@ __global__ void __launch_bounds__(kPartThreads) sample_list_kernel(
   if (!(t > 0.0f)) return;  // greedy row
   const float tp = top_ps[r];
   const Limits lim = limits_of(top_ks[r], tp, cols);
-  if (!lim.truncate) return;
   const float* row = logits + r * ld;
+  if (!lim.truncate) {
+    draw_all(row, cols, q, t, row_max(st, r, t), row_sum(st, r),
+             gumbel_row(seeds[r], positions[r]), st.mass + blockIdx.x, st.count + blockIdx.x);
+    return;
+  }
   // (threshold, part) totals: kParts = 16 lanes per threshold
   static_assert(kParts == 16 && kCuts * kParts <= kPartThreads, "one thread per total");
   if (threadIdx.x < kCuts * kParts) {
@@ -481,8 +574,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_list_kernel(
   }
   if (threadIdx.x == 0) s_n = 0;
   const float mx = row_max(st, r, t);
-  float sum = 0.0f;
-  for (int p = 0; p < kParts; ++p) sum += st.sum[r * kParts + p];
+  const float sum = row_sum(st, r);
   __syncthreads();
   int j = 0;
   while (j < kCuts && !(static_cast<uint64_t>(s_cnt[j]) >= lim.k || s_mass[j] > (tp + 1e-3f) * sum ||
@@ -692,12 +784,15 @@ __global__ void __launch_bounds__(kSampleThreads) sample_select_kernel(
 
   float bv = -INFINITY;
   int64_t bi = cols;
-  if (!(t > 0.0f)) {  // greedy row
+  const Limits lim = limits_of(top_ks[r], top_ps[r], cols);
+  if (!(t > 0.0f) || !lim.truncate) {  // the parts' best logits or draws
     if (tid == 0) {
+      const float* v = t > 0.0f ? st.mass : st.best;
+      const int32_t* i = t > 0.0f ? st.count : st.best_at;
       for (int q = 0; q < kParts; ++q) {
-        const int at = st.best_at[r * kParts + q];
-        if (at < ncols && better(st.best[r * kParts + q], at, bv, bi)) {
-          bv = st.best[r * kParts + q];
+        const int at = i[r * kParts + q];
+        if (at < ncols && better(v[r * kParts + q], at, bv, bi)) {
+          bv = v[r * kParts + q];
           bi = at;
         }
       }
@@ -706,11 +801,9 @@ __global__ void __launch_bounds__(kSampleThreads) sample_select_kernel(
     return;
   }
   const float mx = row_max(st, r, t);
-  float sum = st.sum[r * kParts];
-  for (int q = 1; q < kParts; ++q) sum += st.sum[r * kParts + q];
+  const float sum = row_sum(st, r);
   uint32_t* ws = keys_ws + r * cols;
 
-  const Limits lim = limits_of(top_ks[r], top_ps[r], cols);
   const uint64_t k_lim = lim.k, mass_lim = lim.mass;
   const uint32_t row_hash = gumbel_row(seeds[r], positions[r]);
   auto draw = [&](uint32_t key, int c) {
@@ -724,13 +817,6 @@ __global__ void __launch_bounds__(kSampleThreads) sample_select_kernel(
     block_best(bv, bi, s_bv, s_bi);
     if (tid == 0) out[r] = bi < cols ? bi : 0;
   };
-  if (!lim.truncate) {  // every token kept
-    for_each_col<4>(row, ncols, [&](float v, int c) {
-      draw(__float_as_uint(expf(v / t - mx) / sum), c);
-    });
-    finish();
-    return;
-  }
 
   // The list: every column with e >= kCutMin[cut_at]. A column outside has p at most
   // fl(kCutMin[cut_at] / sum), so a cut key above that lies, with all its ties and everything
@@ -929,12 +1015,12 @@ extern "C" int sid_sample_rows(const float* logits, int64_t ld, const float* tem
     int rc = check_launch("sample_rows max");
     if (rc != SID_OK) return rc;
     hipLaunchKernelGGL(sample_sum_kernel, grid, dim3(kPartThreads), 0, s, lg, ld,
-                       temperatures + r0, (int)cols, st);
+                       temperatures + r0, top_ks + r0, top_ps + r0, (int)cols, st);
     rc = check_launch("sample_rows sum");
     if (rc != SID_OK) return rc;
     hipLaunchKernelGGL(sample_list_kernel, grid, dim3(kPartThreads), 0, s, lg, ld,
-                       temperatures + r0, top_ks + r0, top_ps + r0, (int)cols, st,
-                       lists + r0 * cols);
+                       temperatures + r0, top_ks + r0, top_ps + r0, seeds + r0, positions + r0,
+                       (int)cols, st, lists + r0 * cols);
     rc = check_launch("sample_rows list");
     if (rc != SID_OK) return rc;
     hipLaunchKernelGGL(sample_select_kernel, dim3((unsigned)n), dim3(kSampleThreads),
