@@ -1794,7 +1794,7 @@ extern "C" int sid_linear(const void* x, int64_t ldx, const void* w, const void*
   if (rc != SID_OK) return rc;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   // The streaming kernel reads the weights once per 64-row group; past one group the tile
-  // kernel is faster (M = 128, 151936 x 1024 fp32 logits 165 vs 101 us, identical bits), and
+  // kernel is faster (M = 128, 151936 x 1024 fp32 logits 165 vs 90 us, identical bits), and
   // below kStreamMinN columns at any M: its loads run up to four sub-tiles ahead where the
   // row-group kernel waits for each chunk. Weights from HBM, row group vs tiles, us:
   // 1 x 1024 x 2048 15.4 vs 7.9, 32 x 1024 x 3072 29.9 vs 10.8, 16 x 4096 x 1024 10.6 vs 6.7,
@@ -1840,7 +1840,7 @@ extern "C" int sid_linear_partials(const void* x, int64_t ldx, const void* w, fl
 // sid_linear_argmax: up to one 64-row group streams the weights once (linear_stream_kernel,
 // one candidate per workgroup); more rows take the tiled GEMM with the argmax epilogue (one
 // candidate per 128-column tile, no logits needed: verify pass, 128 rows x 151936,
-// 101 us GEMM + 32 us argmax_rows before). Both reduce with argmax_finalize_kernel. The
+// 85 us; with logits 90 + argmax_rows 32). Both reduce with argmax_finalize_kernel. The
 // workspace holds cu_count() * STREAM_WAVES candidates per row, which bounds the tiled
 // path's column tiles.
 static bool argmax_streams(int64_t m, int64_t n, int64_t k) {
@@ -1931,8 +1931,8 @@ static void launch_sample_mbs(const bf16_t* x, int64_t ldx, const void* w, int m
 // The streaming sampler reads the weights once per 64-row group; above this many rows (or
 // when asked) the tiled GEMM with the sampler epilogue reads them once per 128-row tile
 // (candidate groups: 128-column tiles instead of streaming waves). Measured at T = 0.7,
-// 151936 x 1024, graph-timed (streaming vs tiled, us): 1 row 80 vs 108, 64 rows 120 vs
-// 142, 128 rows 214 vs 158, 192 rows 265 vs 266, 256 rows 285 vs 284.
+// 151936 x 1024, graph-timed (streaming vs tiled, us): 1 row 73 vs 91, 64 rows 108 vs
+// 119, 96 rows 181 vs 132, 128 rows 199 vs 137, 192 rows 291 vs 216, 256 rows 375 vs 238.
 constexpr int64_t kStreamSampleMaxM = 64;
 
 extern "C" int sid_linear_sample(const void* x, int64_t ldx, const void* w, int64_t m, int64_t n,

@@ -62,11 +62,11 @@ def linear_partials(x: torch.Tensor, weight: torch.Tensor,
 
 
 # sid_linear_silu_mul (gate_up projection + SwiGLU in one launch, no projection written)
-# serves every row count at K = 1024: up to 95 rows a kernel in which every workgroup reads
+# serves every row count at K = 1024: up to 32 rows a kernel in which every workgroup reads
 # its rows' whole x for 16 output columns (against the split-K pair it saves a launch and the
-# fp32 partials' round trip: M=1 8.0 -> 5.2 us, M=32 9.9 -> 6.8, M=64 12.5 -> 9.3), from 96
-# rows the tiled GEMM with the SwiGLU in its epilogue (M=128 15.6 -> 12.8 us, M=192
-# 20.7 -> 12.5, M=2048 48.2 -> 38.4 against linear + silu_mul). Same bits everywhere.
+# fp32 partials' round trip: M=1 8.0 -> 5.2 us, M=32 9.9 -> 6.8), from 33 rows the tile GEMM
+# with the SwiGLU in its epilogue (weights from HBM, M=32 7.4 vs 6.6 us, M=64 7.9 vs 8.9, M=95
+# 7.5 vs 12.6; M=8192 95 us). Same bits everywhere.
 def linear_silu_mul_preferred(m: int, k: int) -> bool:
     """Shapes where linear_silu_mul is used for the MLP's first half (K = 1024)."""
     return m >= 1 and k == 1024
