@@ -50,7 +50,7 @@ __device__ __forceinline__ bool better(float v, int64_t i, float bv, int64_t bi)
 // 128 rows 137 vs 113; 256 rows, whose workgroups filled the chip, 151 vs 191). One 1024-thread workgroup per
 // row for everything, nine passes over 151936 columns bound by one CU's latency and LDS
 // atomics, took 205 us for 1 row and 366 for 64 (top-k / top-p mixes over peaked rows); these
-// four take 30 and 72 (max 6 / 11, sum 12 / 30, list 6 / 12, select 9 / 20). Listing in the
+// four take 31 and 69 (max 6 / 11, sum 12 / 30, list 6 / 12, select 9 / 20). Listing in the
 // sum pass at fixed thresholds (three launches): 27 and 173, as rows with top-k alone reach
 // far below the maximum.
 constexpr int kSampleThreads = 1024;
