@@ -473,11 +473,12 @@ __global__ void __launch_bounds__(NW * 64, NW / 2) extend_prefill_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
     const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ qo_indptr,
     const int32_t* __restrict__ kv_indptr, const int32_t* __restrict__ kv_indices,
-    int num_q_heads, int num_kv_heads, int64_t num_slots, float sm_scale, int mtiles,
+    int batch, int num_q_heads, int num_kv_heads, int64_t num_slots, float sm_scale, int mtiles,
     bf16_t* __restrict__ o) {
   extern __shared__ __align__(1024) char lds[];  // [2][K tile, V tile]
   constexpr int ROWS = 8 * NW;  // query positions of the workgroup
   const int b = blockIdx.x;
+  if (b >= batch) return;  // (the grid's padding)
   const int h_kv = blockIdx.y;
   // Late query tiles walk the most keys: dispatch them first.
   const int mtile = mtiles - 1 - static_cast<int>(blockIdx.z);
@@ -676,13 +677,33 @@ __global__ void __launch_bounds__(256) extend_merge_kernel(
 
 // Fan the splits out when the grid would leave most CUs idle.
 constexpr int kFanoutBelowWg = 512;
-// 64-row workgroups in the grid from which they are used (4 per CU of 256).
-constexpr int64_t kWideWg = 1024;
+// Query positions of a prefill workgroup. The 64-row ones (8 waves) load each key tile half as
+// often, but a causal grid ends on its longest ones, and a short request leaves some of their
+// waves idle. They win once the rows that exist (total_q, not batch x longest) fill 2.6 of
+// them per CU of 256 and at least half of the batch x longest rows exist. 32- vs 64-row, us:
+// 1 x 4096 131 vs 152, 2 x 2304 78 vs 85, 1 x 5120 173 vs 180, 3 x 1800 77 vs 70, 2 x 3000
+// 127 vs 113, 4 x 2048 122 vs 116, 1 x 8192 416 vs 380; 12 x 512 36 vs 39, 16 x 512 47 vs 49,
+// 6 x 1024 54 vs 53; 3000 + 40 x 33 80 vs 120, 2048 + 15 x 16 54 vs 80, 1024 + 60 x 120 39 vs
+// 45, 5000 + 3000 229 vs 204.
+constexpr int64_t kWideWg = 672;
+constexpr int kWideMinLen = 1024;
+int prefill_rows(int batch, int64_t total_q, int num_kv_heads, int max_extend_len) {
+  const bool uniform = 2 * total_q >= static_cast<int64_t>(batch) * max_extend_len;
+  return max_extend_len >= kWideMinLen && uniform &&
+                 num_kv_heads * ((total_q + 63) / 64) >= kWideWg
+             ? 64
+             : 32;
+}
 
 }  // namespace
 }  // namespace sid
 
 using namespace sid;
+
+extern "C" int sid_extend_attention_query_rows(int batch, int64_t total_q, int num_kv_heads,
+                                               int max_extend_len) {
+  return prefill_rows(batch, total_q, num_kv_heads, max_extend_len);
+}
 
 extern "C" int64_t sid_extend_attention_workspace_bytes(int batch, int64_t total_q,
                                                         int num_q_heads, int num_kv_heads,
@@ -738,21 +759,20 @@ extern "C" int sid_extend_attention_fwd(const void* q, const void* k_cache, cons
     return check_launch("extend_attention merge");
   }
   SID_REQUIRE(mtiles <= 65535, "extend_attention: grid too large");
-  // 64-row workgroups (8 waves) load each key tile half as often, but a causal grid ends on
-  // its longest ones: from 4 of them per CU and 512 rows they win (4 x 2048 129 vs 136 us,
-  // 8420 ragged tokens 138 vs 154), below that the 32-row ones (1 x 4096 136 vs 148, 1 x 2048
-  // 50 vs 70, 200 x 1 over 1000 keys 153 vs 191).
+  // Request b's workgroups are `batch` ids apart. Where only some requests reach the late tiles
+  // an even distance puts a long request's on few XCDs and CUs, so the grid then has an odd
+  // one (2048 + 15 x 16 445 -> 54 us, 31 x 1 + 4000 3160 -> 126, 5000 + 3000 268 -> 209; full
+  // batches keep theirs: 12 x 512 36 vs 38 padded, 8 x 1024 69 vs 72).
+  const bool ragged = 8 * total_q < 7 * static_cast<int64_t>(batch) * max_extend_len;
   auto prefill = [&](auto kern, int nw) {
     const int mt = ceil_div(max_extend_len, 8 * nw);
-    hipLaunchKernelGGL(kern, dim3(batch, num_kv_heads, mt), dim3(nw * 64), 4 * kTileBytes, s,
-                       (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, qo_indptr,
-                       kv_indptr, kv_indices, num_q_heads, num_kv_heads, num_slots, sm_scale, mt,
-                       (bf16_t*)o);
+    hipLaunchKernelGGL(kern, dim3(ragged ? batch | 1 : batch, num_kv_heads, mt), dim3(nw * 64),
+                       4 * kTileBytes, s, (const bf16_t*)q, (const bf16_t*)k_cache,
+                       (const bf16_t*)v_cache, qo_indptr, kv_indptr, kv_indices, batch, num_q_heads,
+                       num_kv_heads, num_slots, sm_scale, mt, (bf16_t*)o);
   };
   const bool off32 = num_slots * num_kv_heads * D * 2 < (1ll << 32);
-  const bool wide = max_extend_len >= 512 && static_cast<int64_t>(batch) * num_kv_heads *
-                                                     ceil_div(max_extend_len, 64) >= kWideWg;
-  if (wide) {
+  if (prefill_rows(batch, total_q, num_kv_heads, max_extend_len) == 64) {
     off32 ? prefill(extend_prefill_kernel<8, true>, 8) : prefill(extend_prefill_kernel<8, false>, 8);
   } else {
     off32 ? prefill(extend_prefill_kernel<4, true>, 4) : prefill(extend_prefill_kernel<4, false>, 4);

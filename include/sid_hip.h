@@ -196,6 +196,11 @@ int64_t sid_extend_attention_workspace_bytes(int batch, int64_t total_q, int num
                                              int num_kv_heads, int max_extend_len,
                                              int max_kv_len);
 
+/* Query positions per workgroup (32 or 64) of such a call without fan-out: a speed choice, from
+ * the rows that exist (total_q) and the longest request. The results are the same. */
+int sid_extend_attention_query_rows(int batch, int64_t total_q, int num_kv_heads,
+                                    int max_extend_len);
+
 /*
  * out[r] = x[r] * rsqrt(mean(x[r]^2) + eps) * w, fp32 math, bf16 I/O.
  * x, out: bf16 [rows, hidden]; w: bf16 [hidden]; hidden a multiple of 8,

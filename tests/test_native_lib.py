@@ -77,6 +77,16 @@ def test_validation_errors_without_device_work(ext):
                                     None, None, 0, 0, None, None) == 0
 
 
+@pytest.mark.parametrize("lens,rows", [
+    ([2048] * 4, 64), ([4096] * 2, 64), ([8192], 64), ([2300, 1800, 900, 2000, 400, 1020], 64),
+    ([2048], 32), ([512] * 16, 32),
+    # long prompts among short ones: few rows exist of batch x longest
+    ([2048] + [16] * 15, 32), ([3000] + [33] * 40, 32), ([1024] + [120] * 60, 32),
+], ids=lambda v: str(v)[:24])
+def test_prefill_workgroup_follows_the_rows_that_exist(ext, lens, rows):
+    assert ext.lib.sid_extend_attention_query_rows(len(lens), sum(lens), 8, max(lens)) == rows
+
+
 def test_ops_reject_cpu_tensors(ext):
     import torch
     q = torch.zeros(1, 16, 128, dtype=torch.bfloat16)
