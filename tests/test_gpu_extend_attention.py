@@ -142,10 +142,31 @@ def test_split_fanout_bitwise_equals_sequential_fold(specs):
     assert torch.equal(a, c)
 
 
+@pytest.mark.parametrize("prefix,rows,at", [(48, 32, 70), (16, 64, 64), (1000, 40, 1030)])
+def test_hidden_values_do_not_reach_earlier_waves(prefix, rows, at):
+    """An infinite and a NaN V row in a tile that only later waves of the query tile see: fan-out
+    and sequential walk give the same rows, and the waves before it stay finite."""
+    from sid.kernels.jit import load_ext
+    ext = load_ext()
+    print(f"hidden values prefix={prefix} rows={rows} at={at}", flush=True)
+    q, kb, vb, qo, kvp, idx = _make([(prefix, rows)], seed=at)
+    vb[idx[at].long(), :, 5] = float("inf")
+    vb[idx[at].long(), :, 9] = float("nan")
+    kv = prefix + rows
+    ws = torch.empty(ext.extend_attention_workspace_bytes(1, rows, HQ, HKV, rows, kv),
+                     dtype=torch.uint8, device="cuda")
+    a, b = torch.empty_like(q), torch.empty_like(q)
+    ext.extend_attention_fwd(q, kb, vb, qo, kvp, idx, rows, SCALE, a, kv, ws)
+    ext.extend_attention_fwd(q, kb, vb, qo, kvp, idx, rows, SCALE, b, kv, None)
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    before = (at // 64 * 64 - prefix) // 16 * 16  # rows of waves that end before the tile
+    assert before > 0 and torch.isfinite(a[:before]).all()
+
+
 @pytest.mark.parametrize("specs,slots", [
     # 32-row workgroups: one-row requests, tails of 32 rows and 64-key tiles, empty requests
     ([(i % 5, 1 + (37 * i) % 70) for i in range(80)] + [(300, 0)], None),
-    # 64-row workgroups (512 rows and more, at least 1024 of them): ragged around tile edges
+    # 64-row workgroups: ragged around tile edges
     ([(0, 1024), (3, 1023), (0, 961), (17, 960), (0, 512), (255, 65), (0, 64), (1, 1)] +
      [(0, 577 + i) for i in range(4)], None),
     # a pool of more than 4 GiB a side (64-bit row offsets)
