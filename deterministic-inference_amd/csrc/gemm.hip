@@ -314,6 +314,27 @@ __device__ __forceinline__ void sstate_add(SState& a, float vr, int col, float t
   }
 }
 
+// sstate_add to the empty state (the same values without its exponential).
+__device__ __forceinline__ SState sstate_first(float vr, int col, float t, uint32_t h) {
+  SState a = sstate_empty();
+  if (!(t > 0.0f)) {
+    a.v1 = vr;
+    a.i1 = col;
+    return a;
+  }
+  const float xv = vr / t;
+  const bool some = xv > -INFINITY;
+  a.m = some ? xv : -INFINITY;
+  a.s = some ? 1.0f : xv - xv;  // (-inf and NaN: NaN)
+  const float xg = xv + seeded_gumbel(h, col);
+  if (xg >= -INFINITY) {
+    a.v1 = xg;
+    a.x1 = xv;
+    a.i1 = col;
+  }
+  return a;
+}
+
 // a <- a merged with b (a fixed function of the two states).
 __device__ __forceinline__ void sstate_merge(SState& a, const SState& b, bool greedy) {
   if (greedy) {
@@ -735,10 +756,10 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) linear_tile_kernel(
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
-      // lm_head epilogues: each lane's best (EPI_ARGMAX) or sampler state (EPI_SAMPLE) of a
-      // row over its 4 NB columns in increasing order (logits written as fp32 when y is
-      // given), merged over the 4 lanes of the row, then over the WN waves of the row band in
-      // wave order through LDS: one record per (column tile, row).
+      // lm_head epilogues: each lane's best (EPI_ARGMAX) of a row over its 4 NB columns, or its
+      // sampler state (EPI_SAMPLE; logits written as fp32 when y is given), merged over the 4
+      // lanes of the row, then over the WN waves of the row band in wave order through LDS: one
+      // record per (column tile, row).
       float* s_f = reinterpret_cast<float*>(scratch);
       static_assert(6 * WN * TM * 4 <= S::SCRATCH, "statistics exceed the scratch");
       int* s_i = reinterpret_cast<int*>(s_f + 5 * WN * TM);
@@ -755,7 +776,9 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) linear_tile_kernel(
           temp = out.sp.temps[rc];
           h = gumbel_row(out.sp.seeds[rc], out.sp.positions[rc]);
         }
-        SState a = sstate_empty();
+        // Sampler state of each column residue mod 16 (four a lane), in the order that is part of
+        // a row's softmax sum: a residue's columns, then residues r and r ^ 1, ^ 2, ^ 4, ^ 8.
+        SState a = sstate_empty(), c[4] = {a, a, a, a};
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
           const int col = col0 + 16 * j + 4 * eg;
@@ -767,7 +790,11 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) linear_tile_kernel(
             if (EPI == EPI_ARGMAX && out.bias != nullptr) v += bf16_to_f32(out.bias[col + e]);
             q[e] = round_bf16(v);
             if constexpr (EPI == EPI_SAMPLE) {
-              sstate_add(a, q[e], col + e, temp, h);
+              if (j == 0) {
+                c[e] = sstate_first(q[e], col + e, temp, h);
+              } else {
+                sstate_add(c[e], q[e], col + e, temp, h);
+              }
             } else if (argmax_better(q[e], col + e, a.v1, a.i1)) {
               a.v1 = q[e];
               a.i1 = col + e;
@@ -782,6 +809,13 @@ __global__ void __launch_bounds__(WM * WN * 64, OCC) linear_tile_kernel(
               for (int e = 0; e < 4; ++e) y[e] = q[e];
             }
           }
+        }
+        if constexpr (EPI == EPI_SAMPLE) {
+          const bool greedy = !(temp > 0.0f);
+          sstate_merge(c[0], c[1], greedy);
+          sstate_merge(c[2], c[3], greedy);
+          sstate_merge(c[0], c[2], greedy);
+          a = c[0];
         }
         sstate_merge_xor<16, 64>(a, EPI == EPI_ARGMAX || !(temp > 0.0f));
         if (eg == 0) {

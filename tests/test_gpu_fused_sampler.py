@@ -140,3 +140,34 @@ def test_row_limits_per_grouping(lm_head):
     ws = torch.empty(ext.linear_sample_workspace_bytes(257), dtype=torch.uint8, device="cuda")
     with pytest.raises(RuntimeError, match="M <= 256"):
         linear_sample(x, lm_head, temps, seeds, pos, workspace=ws, tiles=False)
+
+
+def test_tile_grouping_order_of_the_softmax_sum():
+    """The order in which a 128-column tile sums its softmax terms is part of a row's token: a
+    column residue mod 16 first, then residues r and r ^ 1, ^ 2, ^ 4, ^ 8, then the tile's two
+    64-column halves. One term of 1 among terms of 2^-25 shows it: a term that meets the 1
+    alone is lost (half an ulp, ties to even), the sums of four and more are not, so the total
+    is 1 + (4 + 8 + 16 + 32) 2^-25 = 1 + 15 * 2^-23."""
+    from sid.kernels.jit import load_ext
+    ext = load_ext()
+    n, m = 384, 70  # (rows in two waves' bands, the last tile's halves alike)
+    temp = 17.25 / (25 * math.log(2)) * (1 - 2e-6)  # exp(-17.25 / temp) just below 2^-25
+    vals = torch.full((n,), -100.0)
+    tops = [0, 128 + 3, 256 + 64 + 9]
+    for top in tops:
+        half = top // 64 * 64
+        vals[half:half + 64] = -17.25
+        vals[top] = 0.0
+    w = torch.zeros(n, K)
+    w[:, 0] = vals
+    x = torch.zeros(m, K)
+    x[:, 0] = 1.0
+    w, x = w.to(torch.bfloat16).cuda(), x.to(torch.bfloat16).cuda()
+    temps = torch.full((m,), temp, device="cuda")
+    ids = torch.arange(m, device="cuda")
+    out = torch.empty(m, dtype=torch.int64, device="cuda")
+    ws = torch.zeros(ext.linear_sample_workspace_bytes(m), dtype=torch.uint8, device="cuda")
+    ext.linear_sample(x, w, temps, ids, ids, ws, out, tiles=True)
+    groups = torch.cuda.get_device_properties(0).multi_processor_count * 8
+    sums = ws.view(torch.float32)[groups * m:2 * groups * m].view(groups, m)[:n // 128]
+    assert torch.equal(sums.cpu(), torch.full((n // 128, m), 1.0 + 15 * 2.0 ** -23))
