@@ -18,7 +18,7 @@
 //   * linear_tile_kernel: direct y (prefill, and decode / verify rows past the split-K cuts),
 //     persistent tiles of four shapes; also gate_up with the SwiGLU epilogue and the lm_head
 //     of more than 64 rows with the argmax or sampler epilogue;
-//   * linear_kernel: direct y for row strides past the tile kernel's 32-bit offsets;
+//   * linear_kernel: direct y (or greedy argmax) for rows past the tile kernel's 32-bit offsets;
 //   * linear_stream_kernel: lm_head-shaped N (persistent grid, x staged once per CU), with
 //     an optional fused greedy argmax.
 #include "common.h"
@@ -99,14 +99,29 @@ __device__ __forceinline__ void chunk_mfma(f32x4_v (&acc)[4], const bf16x8_v (&w
   }
 }
 
+// Greedy argmax order over (value, column), torch's: larger value, then smaller index; NaN
+// above everything, first NaN wins. A total order, so a maximum over any split of the
+// columns into candidates, reduced in any order, is the same (value, column).
+__device__ __forceinline__ bool argmax_better(float v, int i, float bv, int bi) {
+  const bool vn = v != v;
+  const bool bn = bv != bv;
+  if (vn || bn) {
+    if (vn && bn) return i < bi;
+    return vn;
+  }
+  return v > bv || (v == bv && i < bi);
+}
+
 // Direct y = x w^T (+ bias) for one 64-row group and 16*NW columns: every chunk in order,
 // the next chunk's weights and x prefetched into registers during the current chunk's
 // MFMAs. NW waves share one staged x chunk. (Only for sizes that tiles_fit refuses.)
-template <int NW>
+// AM: also each row's best (bf16-rounded logit, column) of the wave's 16 columns, to
+// best_val / best_idx [wave of the grid][M]; y may then be null.
+template <int NW, bool AM>
 __global__ void __launch_bounds__(NW * 64) linear_kernel(
     const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ w,
     const bf16_t* __restrict__ bias, void* __restrict__ y, int64_t M, int64_t N, int64_t K,
-    int out_fp32) {
+    int out_fp32, float* __restrict__ best_val, int* __restrict__ best_idx) {
   __shared__ __align__(16) bf16_t sx[MROWS * XS];
 
   const int nchunks = static_cast<int>(K / KC);
@@ -167,7 +182,25 @@ __global__ void __launch_bounds__(NW * 64) linear_kernel(
           float v = total[mb][i];
           if (bias != nullptr) v += bv;
           const int64_t off = (m0 + row) * N + n0 + col;
-          if (out_fp32) {
+          if constexpr (AM) {  // (the 16 lanes of a row are active together)
+            v = round_bf16(v);
+            if (y != nullptr) static_cast<float*>(y)[off] = v;
+            int ix = static_cast<int>(n0) + col;
+#pragma unroll
+            for (int mask = 1; mask < 16; mask <<= 1) {
+              const float ov = lane_xor(v, mask);
+              const int oi = __builtin_amdgcn_ds_bpermute((lane ^ mask) << 2, ix);
+              if (argmax_better(ov, oi, v, ix)) {
+                v = ov;
+                ix = oi;
+              }
+            }
+            if (r == 0) {
+              const int64_t o = (static_cast<int64_t>(blockIdx.x) * NW + wave) * M + m0 + row;
+              best_val[o] = v;
+              best_idx[o] = ix;
+            }
+          } else if (out_fp32) {
             static_cast<float*>(y)[off] = round_bf16(v);
           } else {
             static_cast<bf16_t*>(y)[off] = f32_to_bf16(v);
@@ -244,19 +277,6 @@ __global__ void __launch_bounds__(NW * 64) linear_chunk_kernel(
       if (row < mrows) dst[static_cast<int64_t>(row) * N] = acc[mb][i];
     }
   }
-}
-
-// Greedy argmax order over (value, column), torch's: larger value, then smaller index; NaN
-// above everything, first NaN wins. A total order, so a maximum over any split of the
-// columns into candidates, reduced in any order, is the same (value, column).
-__device__ __forceinline__ bool argmax_better(float v, int i, float bv, int bi) {
-  const bool vn = v != v;
-  const bool bn = bv != bv;
-  if (vn || bn) {
-    if (vn && bn) return i < bi;
-    return vn;
-  }
-  return v > bv || (v == bv && i < bi);
 }
 
 struct SampleStats {
@@ -1840,8 +1860,9 @@ extern "C" int sid_linear(const void* x, int64_t ldx, const void* w, const void*
     launch_tiles<EPI_Y>(x, ldx, w, m, n, k, tile_out(y, bias, out_fp32), s);
   } else {
     const dim3 grid((unsigned)(n / 64), 1u, (unsigned)((m + MROWS - 1) / MROWS));
-    hipLaunchKernelGGL((linear_kernel<4>), grid, dim3(256), 0, s, (const bf16_t*)x, ldx,
-                       (const bf16_t*)w, (const bf16_t*)bias, y, m, n, k, out_fp32);
+    hipLaunchKernelGGL((linear_kernel<4, false>), grid, dim3(256), 0, s, (const bf16_t*)x, ldx,
+                       (const bf16_t*)w, (const bf16_t*)bias, y, m, n, k, out_fp32, nullptr,
+                       nullptr);
   }
   return check_launch("linear");
 }
@@ -1911,12 +1932,19 @@ extern "C" int sid_linear_argmax(const void* x, int64_t ldx, const void* w, cons
     launch_stream<true>(x, ldx, w, bias, logits, static_cast<int>(m), static_cast<int>(n), 1, bv,
                         bi, s);
     used = cu_count();
+  } else if (k >= (1ll << 23)) {
+    // Weight rows past the tile kernel's 32-bit offsets; one candidate per 16 columns.
+    SID_REQUIRE(n / 16 <= cands, "linear_argmax: N=%lld has more than %lld column blocks",
+                (long long)n, (long long)cands);
+    const dim3 grid((unsigned)(n / 64), 1u, (unsigned)((m + MROWS - 1) / MROWS));
+    hipLaunchKernelGGL((linear_kernel<4, true>), grid, dim3(256), 0, s, (const bf16_t*)x, ldx,
+                       (const bf16_t*)w, (const bf16_t*)bias, logits, m, n, k, 1, bv, bi);
+    used = static_cast<int>(n / 16);
   } else {
     const int64_t tiles = (n + 127) / 128;
     SID_REQUIRE(tiles <= cands, "linear_argmax: N=%lld has more than %lld column tiles",
                 (long long)n, (long long)cands);
     SID_REQUIRE((m + 127) / 128 <= 65535, "linear_argmax: too many rows");
-    SID_REQUIRE(k < (1ll << 23), "linear_argmax: K too large");
     TileOut out = tile_out(logits, bias, 1);
     out.best_val = bv;
     out.best_idx = bi;

@@ -243,3 +243,34 @@ def test_wide_row_strides(m, ldx):
     ws = torch.empty(ext.linear_argmax_workspace_bytes(m), device="cuda", dtype=torch.uint8)
     ext.linear_argmax(x, w, None, logits, ws, out)
     assert torch.equal(logits, ref) and torch.equal(out, ref.argmax(1))
+
+
+@pytest.mark.parametrize("m,n", [(1, 64), (3, 128)])
+def test_weight_rows_past_32_bit_offsets(m, n):
+    """K of 2^23, where a tile's weight rows reach past 32-bit offsets: sid_linear's bits against
+    the split-K chunks folded in order, and the greedy head's logits and tokens against them."""
+    from sid.kernels.jit import load_ext
+    ext = load_ext()
+    k = 1 << 23
+    print(f"long weight rows m={m} n={n} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(m, k, device="cuda", generator=g).to(torch.bfloat16)
+    w = torch.empty(n, k, device="cuda", dtype=torch.bfloat16)
+    for row in w:  # (a row at a time: no second copy of the weights in float)
+        row.copy_(torch.randn(k, device="cuda", generator=g) * 0.05)
+    b = torch.randn(n, device="cuda", generator=g).to(torch.bfloat16)
+    part = torch.empty(k // 256, m, n, device="cuda", dtype=torch.float32)
+    ext.linear_partials(x, w, part)
+    fold = part[0].clone()
+    for c in part[1:]:
+        fold += c
+    ref = (fold + b.float()).to(torch.bfloat16).float()
+    y = torch.empty(m, n, device="cuda", dtype=torch.float32)
+    ext.linear(x, w, b, y, True)
+    assert torch.equal(y, ref)
+    ws = torch.empty(ext.linear_argmax_workspace_bytes(m), device="cuda", dtype=torch.uint8)
+    for logits in (torch.empty_like(y), None):
+        out = torch.full((m,), -1, device="cuda", dtype=torch.int64)
+        ext.linear_argmax(x, w, b, logits, ws, out)
+        assert torch.equal(out, ref.argmax(1))
+        assert logits is None or torch.equal(logits, ref)
