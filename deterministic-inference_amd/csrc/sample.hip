@@ -953,6 +953,12 @@ __global__ void __launch_bounds__(kSampleThreads) sample_select_kernel(
   finish();
 }
 
+// A launch holds fewer than 2^32 work-items (beyond that rows are silently left out).
+constexpr int64_t kRowsPerLaunch = 1 << 19;
+static_assert(kRowsPerLaunch * kParts * kPartThreads < (1ll << 32) &&
+                  kRowsPerLaunch * kSampleThreads < (1ll << 32),
+              "a launch's work-items");
+
 }  // namespace
 }  // namespace sid
 
@@ -966,11 +972,15 @@ extern "C" int sid_argmax_rows(const float* logits, int64_t ld, int64_t* out, in
   SID_REQUIRE(cols > 0 && ld >= cols, "argmax_rows: bad row stride %lld for %lld columns",
               (long long)ld, (long long)cols);
   SID_REQUIRE(rows < (1ll << 31) && cols < (1ll << 31), "argmax_rows: too large");
-  hipLaunchKernelGGL(argmax_kernel, dim3((unsigned)rows), dim3(kSampleThreads), 0,
-                     static_cast<hipStream_t>(stream), logits, ld, out, cols);
-  return check_launch("argmax_rows");
+  for (int64_t r0 = 0; r0 < rows; r0 += kRowsPerLaunch) {
+    hipLaunchKernelGGL(argmax_kernel, dim3((unsigned)std::min(kRowsPerLaunch, rows - r0)),
+                       dim3(kSampleThreads), 0, static_cast<hipStream_t>(stream), logits + r0 * ld,
+                       ld, out + r0, cols);
+    const int rc = check_launch("argmax_rows");
+    if (rc != SID_OK) return rc;
+  }
+  return SID_OK;
 }
-
 
 // Per row: one word per column (the listed columns, or every column's key), then the parts'
 // statistics.
@@ -1001,7 +1011,6 @@ extern "C" int sid_sample_rows(const float* logits, int64_t ld, const float* tem
   const int64_t parts = rows * kParts;
   hipFuncSetAttribute(reinterpret_cast<const void*>(&sample_select_kernel),
                       hipFuncAttributeMaxDynamicSharedMemorySize, kSelectLds + kListHistLds);
-  constexpr int64_t kRowsPerLaunch = 1 << 24;  // kParts workgroups a row in a 31-bit grid
   for (int64_t r0 = 0; r0 < rows; r0 += kRowsPerLaunch) {
     const int64_t n = std::min(kRowsPerLaunch, rows - r0);
     const float* lg = logits + r0 * ld;

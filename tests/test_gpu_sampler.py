@@ -169,3 +169,33 @@ def test_list_and_full_paths_vs_exact_oracle(vocab):
     print(f"vocab={vocab} rows={m}", flush=True)
     t, k, p = (list(x) for x in zip(*cfg))
     _check(torch.stack(rows), t, k, p, [17 * i + 5 for i in range(m)], [31 * i for i in range(m)])
+
+
+@pytest.mark.parametrize("temp", [1.0425, 1.0495, 1.1])
+def test_forced_token_of_the_largest_float(temp):
+    """A row whose only likely column holds the largest float, as a forced token does: drawn
+    under any limit, also where maximum / T * T rounds to infinity (the first two)."""
+    v = 5000
+    row = torch.full((3, v), -math.inf)
+    row[0, 4321] = row[1, 17] = row[2, 4999] = torch.finfo(torch.float32).max
+    row[1] = row[1].clamp(min=torch.finfo(torch.float32).min)
+    cfg = ([temp] * 3, [20, 50, -1], [1.0, 0.9, 0.5], [1, 2, 3], [7, 8, 9])
+    got = _sample(row, *cfg)
+    assert got.tolist() == sample_exact_ref(row, *cfg).tolist() == [4321, 17, 4999]
+
+
+def test_more_rows_than_one_launch_takes():
+    """A million rows and more: 16 workgroups of 256 threads a row would pass a launch's 2^32
+    work-items, as one of 1024 would for four million."""
+    from sid.kernels.ops import argmax_rows, sample_rows
+    n, v = (1 << 20) + 3, 4
+    print(f"sampler rows={n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    logits = torch.randn(n, v, generator=g, device="cuda")
+    temps = (torch.arange(n, device="cuda") % 3 != 0).float()  # every third row greedy
+    ids = torch.arange(n, device="cuda")
+    got = sample_rows(logits, temps, torch.ones(n, dtype=torch.int64, device="cuda"),
+                          torch.ones(n, device="cuda"), ids, ids)
+    assert torch.equal(got, logits.argmax(1))  # top-k 1: the argmax for every row
+    logits = torch.randn((1 << 22) + 3, 2, generator=g, device="cuda")
+    assert torch.equal(argmax_rows(logits), logits.argmax(1))
