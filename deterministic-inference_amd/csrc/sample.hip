@@ -37,22 +37,24 @@ __device__ __forceinline__ bool better(float v, int64_t i, float bv, int64_t bi)
 // histograms of (count, fixed-point mass), descends to the key of the last kept rank; the
 // tie position among equal keys follows from the index order.
 //
-// Four launches. The first three spread a row over kParts workgroups, one per wave of the
-// 1024-thread column layout for_each_col defines: sample_max_kernel takes the maximum,
-// sample_sum_kernel the sum of exp(x - max) (each of the 1024 layout threads' chains in its
-// own order, so the bits are those of one 1024-thread workgroup) with the number and mass of
-// the columns above a few thresholds, sample_list_kernel lists the columns above the first
-// threshold that should hold the cut. sample_select_kernel, one workgroup per row, finds the
-// cut and draws over the list in LDS: tens to thousands of keys instead of the vocabulary.
-// Rows whose cut is not provably among 16384 columns (flat distributions, non-finite sums)
-// take the passes over all columns there; rows without limits draw in the third launch, part
-// by part (one 1024-thread workgroup per row vs now, us: 1 row 123 vs 40, 64 rows 132 vs 68,
-// 128 rows 137 vs 113; 256 rows, whose workgroups filled the chip, 151 vs 191). One 1024-thread workgroup per
-// row for everything, nine passes over 151936 columns bound by one CU's latency and LDS
-// atomics, took 205 us for 1 row and 366 for 64 (top-k / top-p mixes over peaked rows); these
-// four take 31 and 69 (max 6 / 11, sum 12 / 30, list 6 / 12, select 9 / 20). Listing in the
-// sum pass at fixed thresholds (three launches): 27 and 173, as rows with top-k alone reach
-// far below the maximum.
+// Two forms with the same bits. Few long rows take four launches: the first three spread a row
+// over kParts workgroups, one per wave of the 1024-thread column layout for_each_col defines:
+// sample_max_kernel takes the maximum, sample_sum_kernel the sum of exp(x - max) (each of the
+// 1024 layout threads' chains in its own order, so the bits are those of one 1024-thread
+// workgroup) with the number and mass of the columns above a few thresholds,
+// sample_list_kernel lists the columns above the first threshold that should hold the cut, or
+// draws part by part from a row without limits. sample_select_kernel<false>, one workgroup
+// per row, finds the cut and draws over the list in LDS: tens to thousands of keys instead of
+// the vocabulary. Rows whose cut is not provably among kListCap columns (flat distributions,
+// non-finite sums) take the passes over all columns there. Top-k / top-p mixes over peaked
+// rows of 151936 columns: 1 row 31 us, 64 rows 69 (max 6 / 11, sum 12 / 30, list 6 / 12, select
+// 9 / 20); nine passes over all columns by one workgroup per row took 205 and 366. Listing in
+// the sum pass at fixed thresholds (three launches): 27 and 173, as rows with top-k alone
+// reach far below the maximum.
+//
+// Many rows, or short ones, take sample_select_kernel<true> alone, a workgroup per row for
+// everything: the chip is full without the parts, and greedy and unlimited rows don't pay for
+// launches and early exits they don't need. See one_workgroup_per_row for both sides' times.
 constexpr int kSampleThreads = 1024;
 constexpr int kSampleWaves = kSampleThreads / 64;
 constexpr double kMassUnit = 281474976710656.0;  // 2^48
@@ -143,6 +145,19 @@ __device__ __forceinline__ void block_best(float& bv, int64_t& bi, float* s_v, i
       bi = s_i[w];
     }
   }
+}
+
+// Every thread's x folded by f: over each wave's lanes, then over the waves in order; every
+// thread gets the result.
+template <typename F>
+__device__ __forceinline__ float block_fold(float x, float* s_v, F&& f) {
+  for (int mask = 1; mask < 64; mask <<= 1) x = f(x, lane_xor(x, mask));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) s_v[threadIdx.x >> 6] = x;
+  __syncthreads();
+  x = s_v[0];
+  for (int w = 1; w < kSampleWaves; ++w) x = f(x, s_v[w]);
+  return x;
 }
 
 // Greedy argmax of one row per workgroup.
@@ -334,6 +349,24 @@ __device__ __forceinline__ Limits limits_of(int64_t k, float tp, int64_t cols) {
   return l;
 }
 
+// The first threshold that should hold the row's cut, by its count, or by its mass with a
+// margin (one that does not is found out by the select); kCuts: none, or more columns than a
+// list takes, or sums that are not finite.
+__device__ __forceinline__ int list_cut(const int* cnt, const float* mass, const Limits& lim,
+                                        float top_p, float sum, int cols) {
+  int j = 0;
+  while (j < kCuts && !(static_cast<uint64_t>(cnt[j]) >= lim.k ||
+                        mass[j] > (top_p + 1e-3f) * sum || cnt[j] == cols))
+    ++j;
+  return j < kCuts && cnt[j] <= kListCap && sum < INFINITY ? j : kCuts;
+}
+
+// A little below the smallest logit with exp(x / t - mx) >= floor.
+__device__ __forceinline__ float list_min(float floor, float t, float mx) {
+  const float ln = logf(floor) - 1e-3f;
+  return t * (mx + ln) - 1e-5f * (fabsf(t * mx) - t * ln);
+}
+
 __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
     const float* __restrict__ logits, int64_t ld, const float* __restrict__ temps,
     const int64_t* __restrict__ top_ks, const float* __restrict__ top_ps, int cols, PartStats st) {
@@ -454,8 +487,8 @@ __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
 }
 
 // A row without limits: the best draw over the part's columns. e / sum as quot: exact to the
-// bit wherever it reaches 2^-59, and below that p + 1e-10 is 1e-10 either way. (In the select,
-// one workgroup per row drew over all columns: 1 row 114 us in all, 256 rows 225.)
+// bit wherever it reaches 2^-59, and below that p + 1e-10 is 1e-10 either way. (1 row 38 us in
+// all, against 104 by one workgroup per row.)
 __device__ __forceinline__ void draw_all(const float* __restrict__ row, int cols, int q, float t,
                                          float mx, float sum, uint32_t row_hash, float* best,
                                          int32_t* best_at) {
@@ -534,10 +567,8 @@ __device__ __forceinline__ void draw_all(const float* __restrict__ row, int cols
 
 // (bound: one read of the logits from L2 / the last-level cache and the launch; sum: also ~45
 // VALU operations an element, 30 us at 64 rows.)
-// The columns of the part with e >= kCutMin[j], for the first threshold j that should hold the
-// row's cut by its count, or by its mass with a margin (one that does not is found out by the
-// select). Candidates are picked by the logit itself, a little below the threshold; only
-// those take an exponential.
+// The columns of the part with e >= kCutMin[j], j = list_cut. Candidates are picked by the
+// logit itself, a little below the threshold; only those take an exponential.
 __global__ void __launch_bounds__(kPartThreads) sample_list_kernel(
     const float* __restrict__ logits, int64_t ld, const float* __restrict__ temps,
     const int64_t* __restrict__ top_ks, const float* __restrict__ top_ps,
@@ -576,18 +607,13 @@ __global__ void __launch_bounds__(kPartThreads) sample_list_kernel(
   const float mx = row_max(st, r, t);
   const float sum = row_sum(st, r);
   __syncthreads();
-  int j = 0;
-  while (j < kCuts && !(static_cast<uint64_t>(s_cnt[j]) >= lim.k || s_mass[j] > (tp + 1e-3f) * sum ||
-                        s_cnt[j] == cols))
-    ++j;
-  if (j < kCuts && !(s_cnt[j] <= kListCap && sum < INFINITY)) j = kCuts;  // (NaN: no list)
+  const int j = list_cut(s_cnt, s_mass, lim, tp, sum, cols);
   if (q == 0 && threadIdx.x == 0) st.cut_at[r * kParts] = j;
   if (j == kCuts) return;
   const PartCols pc = part_cols(row, cols, q);
   uint32_t* list = lists + r * cols + pc.list0;
   const float floor = kCutMin[j];
-  const float ln = logf(floor) - 1e-3f;
-  const float v_min = t * (mx + ln) - 1e-5f * (fabsf(t * mx) - t * ln);
+  const float v_min = list_min(floor, t, mx);
   const Quot div = quot_of(t);
   auto take = [&](float v, int c, bool valid) {
     if (__builtin_amdgcn_ballot_w64(valid && v >= v_min) == 0) return;
@@ -762,6 +788,9 @@ constexpr int kSelectLds = kListCap * 8;                          // keys and co
 static_assert(kHistCopies * 257 * 12 <= kSelectLds, "the full passes' histograms fit there");
 constexpr int kListHistLds = kListCopies * 257 * 12 + 8;
 
+// WHOLE: the one launch of a call; the row's maximum, sum and list are made here, with the
+// bits and in the order of the launches above, and rows of any kind are finished.
+template <bool WHOLE>
 __global__ void __launch_bounds__(kSampleThreads) sample_select_kernel(
     const float* __restrict__ logits, int64_t ld, const float* __restrict__ temps,
     const int64_t* __restrict__ top_ks, const float* __restrict__ top_ps,
@@ -773,7 +802,9 @@ __global__ void __launch_bounds__(kSampleThreads) sample_select_kernel(
   __shared__ int64_t s_scan[kSampleThreads];
   __shared__ uint64_t s_sel[4];
   __shared__ int64_t s_cut;
-  __shared__ int s_ties;
+  __shared__ int s_ties, s_listed;
+  __shared__ int s_cnt[kSampleWaves][kCuts];
+  __shared__ float s_mass[kSampleWaves][kCuts];
   __shared__ uint32_t s_few_key[kFewKeys], s_few_col[kFewKeys];
 
   const int64_t r = blockIdx.x;
@@ -785,7 +816,7 @@ __global__ void __launch_bounds__(kSampleThreads) sample_select_kernel(
   float bv = -INFINITY;
   int64_t bi = cols;
   const Limits lim = limits_of(top_ks[r], top_ps[r], cols);
-  if (!(t > 0.0f) || !lim.truncate) {  // the parts' best logits or draws
+  if (!WHOLE && (!(t > 0.0f) || !lim.truncate)) {  // the parts' best logits or draws
     if (tid == 0) {
       const float* v = t > 0.0f ? st.mass : st.best;
       const int32_t* i = t > 0.0f ? st.count : st.best_at;
@@ -800,50 +831,124 @@ __global__ void __launch_bounds__(kSampleThreads) sample_select_kernel(
     }
     return;
   }
-  const float mx = row_max(st, r, t);
-  const float sum = row_sum(st, r);
   uint32_t* ws = keys_ws + r * cols;
-
   const uint64_t k_lim = lim.k, mass_lim = lim.mass;
   const uint32_t row_hash = gumbel_row(seeds[r], positions[r]);
-  auto draw = [&](uint32_t key, int c) {
-    const float s = logf(__uint_as_float(key) + kSampleEps) + seeded_gumbel(row_hash, c);
+  const Quot by_t = quot_of(t);
+  auto take = [&](float s, int c) {
     if (better(s, c, bv, bi)) {
       bv = s;
       bi = c;
     }
+  };
+  auto draw = [&](uint32_t key, int c) {
+    take(logf(__uint_as_float(key) + kSampleEps) + seeded_gumbel(row_hash, c), c);
   };
   auto finish = [&]() {
     block_best(bv, bi, s_bv, s_bi);
     if (tid == 0) out[r] = bi < cols ? bi : 0;
   };
 
+  float mx, sum;
+  int cut_at;
+  if constexpr (WHOLE) {
+    if (!(t > 0.0f)) {  // greedy row
+      for_each_col<8>(row, ncols, take);
+      finish();
+      return;
+    }
+    float m = -INFINITY;
+    for_each_col<8>(row, ncols, [&](float v, int) { m = fmaxf(m, v); });
+    mx = block_fold(m, s_bv, [](float x, float y) { return fmaxf(x, y); }) / t;
+    float part = 0.0f;
+    int n_cut[kCuts] = {};
+    float m_cut[kCuts] = {};
+    for_each_col<4>(row, ncols, [&](float v, int) {
+      const float e = expf(quot(v, by_t) - mx);
+      part += e;
+      if (lim.truncate && __builtin_amdgcn_ballot_w64(e >= kCutMin[kCuts - 1]) != 0) {
+#pragma unroll
+        for (int j = 0; j < kCuts; ++j) {
+          n_cut[j] += e >= kCutMin[j];
+          m_cut[j] += e >= kCutMin[j] ? e : 0.0f;
+        }
+      }
+    });
+    sum = block_fold(part, s_bv, [](float x, float y) { return x + y; });
+    if (!lim.truncate) {  // (e / sum as quot: see draw_all)
+      const Quot inv = quot_of(sum);
+      for_each_col<4>(row, ncols, [&](float v, int c) {
+        draw(__float_as_uint(quot(expf(quot(v, by_t) - mx), inv)), c);
+      });
+      finish();
+      return;
+    }
+    for (int j = 0; j < kCuts; ++j) {
+      for (int mask = 1; mask < 64; mask <<= 1) {
+        n_cut[j] += __shfl_xor(n_cut[j], mask);
+        m_cut[j] += lane_xor(m_cut[j], mask);
+      }
+      if ((tid & 63) == 0) {
+        s_cnt[tid >> 6][j] = n_cut[j];
+        s_mass[tid >> 6][j] = m_cut[j];
+      }
+    }
+    __syncthreads();
+    if (tid < kCuts) {
+      for (int w = 1; w < kSampleWaves; ++w) {
+        s_cnt[0][tid] += s_cnt[w][tid];
+        s_mass[0][tid] += s_mass[w][tid];
+      }
+    }
+    if (tid == 0) s_listed = 0;
+    __syncthreads();
+    cut_at = list_cut(s_cnt[0], s_mass[0], lim, top_ps[r], sum, ncols);
+  } else {
+    mx = row_max(st, r, t);
+    sum = row_sum(st, r);
+    cut_at = st.cut_at[r * kParts];
+  }
+
   // The list: every column with e >= kCutMin[cut_at]. A column outside has p at most
   // fl(kCutMin[cut_at] / sum), so a cut key above that lies, with all its ties and everything
   // kept, inside, provided that the list does not end before the limits are reached.
-  const int cut_at = st.cut_at[r * kParts];
   if (cut_at < kCuts) {
     uint32_t* l_key = reinterpret_cast<uint32_t*>(s_mem);
     uint32_t* l_col = l_key + kListCap;
     uint64_t* lh_mass = reinterpret_cast<uint64_t*>(s_mem + kSelectLds);
     const Hist lh{lh_mass, reinterpret_cast<uint32_t*>(lh_mass + kListCopies * 257), kListCopies};
-    // Wave w reads part w's list.
-    const int32_t* counts = st.count + st.stride * cut_at + r * kParts;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int n = 0, first = 0;
-    for (int q = 0; q < kParts; ++q) {
-      if (q == wave) first = n;
-      n += counts[q];
+    int n = 0;
+    if constexpr (WHOLE) {
+      n = s_cnt[0][cut_at];
+      const float floor = kCutMin[cut_at];
+      const float v_min = list_min(floor, t, mx);
+      for_each_col<8>(row, ncols, [&](float v, int c) {
+        if (v < v_min) return;
+        const float e = expf(quot(v, by_t) - mx);
+        if (e >= floor) {
+          const int at = atomicAdd(&s_listed, 1);
+          l_col[min(at, kListCap - 1)] = c;
+          l_key[min(at, kListCap - 1)] = __float_as_uint(e / sum);
+        }
+      });
+    } else {
+      // Wave w reads part w's list.
+      const int32_t* counts = st.count + st.stride * cut_at + r * kParts;
+      const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+      int first = 0;
+      for (int q = 0; q < kParts; ++q) {
+        if (q == wave) first = n;
+        n += counts[q];
+      }
+      const uint32_t* list = ws + part_cols(row, ncols, wave).list0;
+#pragma unroll 4
+      for (int i = tid & 63; i < counts[wave]; i += 64) {
+        const uint32_t c = min(list[i], static_cast<uint32_t>(ncols - 1));
+        l_col[first + i] = c;
+        l_key[first + i] = __float_as_uint(expf(quot(row[c], by_t) - mx) / sum);
+      }
     }
     if (tid == 0) s_ties = 0;
-    const uint32_t* list = ws + part_cols(row, ncols, wave).list0;
-    const Quot by_t = quot_of(t);
-#pragma unroll 4
-    for (int i = tid & 63; i < counts[wave]; i += 64) {
-      const uint32_t c = min(list[i], static_cast<uint32_t>(ncols - 1));
-      l_col[first + i] = c;
-      l_key[first + i] = __float_as_uint(expf(quot(row[c], by_t) - mx) / sum);
-    }
     __syncthreads();
     // The select narrows the cut to at most kFewKeys keys; one wave ranks those directly (by
     // key, then column: ties need no separate step). More equal keys than that: the passes
@@ -959,6 +1064,23 @@ static_assert(kRowsPerLaunch * kParts * kPartThreads < (1ll << 32) &&
                   kRowsPerLaunch * kSampleThreads < (1ll << 32),
               "a launch's work-items");
 
+// The rule between the forms (see the top of the file): from 144 rows, 9 / 16 of the CUs, and
+// from fewer where rows are short, as three launches' cost does not shrink with them. One
+// launch vs four, us; greedy rows / rows without limits / top-p 0.9 over peaked rows:
+//   151936 columns:  64 rows  29 vs  23   112 vs  67    70 vs  58
+//                   128       30 vs  35   116 vs 112    76 vs  94
+//                   256       34 vs  55   129 vs 190    85 vs 152
+//   65536 columns:   64       15 vs  15    49 vs  34    36 vs  34
+//                   128       16 vs  21    51 vs  55    37 vs  52
+//   32000 columns:   64       10 vs  13    29 vs  27    27 vs  30
+//                   128       10 vs  16    30 vs  38    26 vs  39
+//   16000 columns:    1        7 vs  11    18 vs  17    16 vs  19
+//    4096 columns:    1        5 vs  11     9 vs  16    13 vs  18
+//                  1024       19 vs  63    36 vs 155    59 vs 169
+bool one_workgroup_per_row(int64_t rows, int64_t cols) {
+  return (144 - rows) * cols <= 144ll * 16000;
+}
+
 }  // namespace
 }  // namespace sid
 
@@ -1009,7 +1131,9 @@ extern "C" int sid_sample_rows(const float* logits, int64_t ld, const float* tem
   uint32_t* lists = static_cast<uint32_t*>(workspace);
   float* stats = reinterpret_cast<float*>(lists + rows * cols);
   const int64_t parts = rows * kParts;
-  hipFuncSetAttribute(reinterpret_cast<const void*>(&sample_select_kernel),
+  const bool whole = one_workgroup_per_row(rows, cols);
+  auto select = whole ? &sample_select_kernel<true> : &sample_select_kernel<false>;
+  hipFuncSetAttribute(reinterpret_cast<const void*>(select),
                       hipFuncAttributeMaxDynamicSharedMemorySize, kSelectLds + kListHistLds);
   for (int64_t r0 = 0; r0 < rows; r0 += kRowsPerLaunch) {
     const int64_t n = std::min(kRowsPerLaunch, rows - r0);
@@ -1018,24 +1142,26 @@ extern "C" int sid_sample_rows(const float* logits, int64_t ld, const float* tem
     const PartStats st{s0, reinterpret_cast<int32_t*>(s0 + parts), s0 + 2 * parts,
                        reinterpret_cast<int32_t*>(s0 + 3 * parts), s0 + (3 + kCuts) * parts, parts,
                        reinterpret_cast<int32_t*>(s0 + (3 + 2 * kCuts) * parts)};
-    const dim3 grid((unsigned)(n * kParts));
-    hipLaunchKernelGGL(sample_max_kernel, grid, dim3(kPartThreads), 0, s, lg, ld,
-                       temperatures + r0, (int)cols, st);
-    int rc = check_launch("sample_rows max");
-    if (rc != SID_OK) return rc;
-    hipLaunchKernelGGL(sample_sum_kernel, grid, dim3(kPartThreads), 0, s, lg, ld,
-                       temperatures + r0, top_ks + r0, top_ps + r0, (int)cols, st);
-    rc = check_launch("sample_rows sum");
-    if (rc != SID_OK) return rc;
-    hipLaunchKernelGGL(sample_list_kernel, grid, dim3(kPartThreads), 0, s, lg, ld,
-                       temperatures + r0, top_ks + r0, top_ps + r0, seeds + r0, positions + r0,
-                       (int)cols, st, lists + r0 * cols);
-    rc = check_launch("sample_rows list");
-    if (rc != SID_OK) return rc;
-    hipLaunchKernelGGL(sample_select_kernel, dim3((unsigned)n), dim3(kSampleThreads),
-                       kSelectLds + kListHistLds, s, lg, ld, temperatures + r0, top_ks + r0,
-                       top_ps + r0, seeds + r0, positions + r0, cols, st, lists + r0 * cols,
-                       out + r0);
+    int rc = SID_OK;
+    if (!whole) {
+      const dim3 grid((unsigned)(n * kParts));
+      hipLaunchKernelGGL(sample_max_kernel, grid, dim3(kPartThreads), 0, s, lg, ld,
+                         temperatures + r0, (int)cols, st);
+      rc = check_launch("sample_rows max");
+      if (rc != SID_OK) return rc;
+      hipLaunchKernelGGL(sample_sum_kernel, grid, dim3(kPartThreads), 0, s, lg, ld,
+                         temperatures + r0, top_ks + r0, top_ps + r0, (int)cols, st);
+      rc = check_launch("sample_rows sum");
+      if (rc != SID_OK) return rc;
+      hipLaunchKernelGGL(sample_list_kernel, grid, dim3(kPartThreads), 0, s, lg, ld,
+                         temperatures + r0, top_ks + r0, top_ps + r0, seeds + r0, positions + r0,
+                         (int)cols, st, lists + r0 * cols);
+      rc = check_launch("sample_rows list");
+      if (rc != SID_OK) return rc;
+    }
+    hipLaunchKernelGGL(select, dim3((unsigned)n), dim3(kSampleThreads), kSelectLds + kListHistLds, s,
+                       lg, ld, temperatures + r0, top_ks + r0, top_ps + r0, seeds + r0,
+                       positions + r0, cols, st, lists + r0 * cols, out + r0);
     rc = check_launch("sample_rows");
     if (rc != SID_OK) return rc;
   }

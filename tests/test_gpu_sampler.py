@@ -199,3 +199,36 @@ def test_more_rows_than_one_launch_takes():
     assert torch.equal(got, logits.argmax(1))  # top-k 1: the argmax for every row
     logits = torch.randn((1 << 22) + 3, 2, generator=g, device="cuda")
     assert torch.equal(argmax_rows(logits), logits.argmax(1))
+
+
+@pytest.mark.parametrize("vocab", [151936, 65537, 20002])
+def test_few_rows_draw_as_among_many(vocab):
+    """A few long rows take four launches, many rows one (a workgroup per row): the same tokens
+    for greedy, unlimited and limited rows, peaked, flat (past the list), tied and non-finite
+    ones, on and off 16-byte alignment."""
+    g = torch.Generator().manual_seed(vocab)
+    n = lambda *s: torch.randn(*s, generator=g)
+    peaked = n(vocab) * 2.0
+    peaked[torch.randint(0, vocab, (40,), generator=g)] += 11.0
+    tied = torch.full((vocab,), -3.0)
+    tied[::7] = 2.0
+    bad = n(vocab)
+    bad[vocab // 2] = math.nan
+    inf = n(vocab)
+    inf[vocab // 3] = math.inf
+    masked = n(vocab) * 3.0
+    masked[torch.randperm(vocab, generator=g)[:vocab * 9 // 10]] = -math.inf
+    limits = [(0.0, 5, 0.5), (0.7, -1, 1.0), (0.7, 20, 0.95), (1.3, -1, 0.9), (1.0, 50, 1.0),
+              (1.0, 12000, 1.0)]
+    rows = [(r, t, k, p) for r in (peaked, n(vocab) * 0.3, tied, masked) for t, k, p in limits]
+    rows += [(r, t, k, p) for r in (bad, inf) for t, k, p in limits[:2]]
+    few = len(rows)
+    assert (144 - few) * vocab > 144 * 16000  # four launches
+    logits = torch.stack([r[0] for r in rows]).to(torch.bfloat16).float()
+    t, k, p = (torch.tensor([r[i] for r in rows]) for i in (1, 2, 3))
+    ids = torch.arange(few)
+    want = _sample(logits, t, k, p, 17 * ids + 5, 31 * ids)
+    at = torch.arange(160) % few  # one launch
+    got = _sample(logits.cuda()[at.cuda()], t[at], k[at], p[at], (17 * ids + 5)[at],
+                  (31 * ids)[at])
+    assert torch.equal(got, want[at])
