@@ -116,7 +116,8 @@ __device__ __forceinline__ void for_each_col(const float* __restrict__ row, int 
     }
     vec = 4 * n4;
   }
-  for (int c = vec + tid; c < cols; c += kSampleThreads) f(row[c], c);
+  for (uint32_t c = vec + tid; c < static_cast<uint32_t>(cols); c += kSampleThreads)
+    f(row[c], static_cast<int>(c));
 }
 
 // Best (value, index) of the block under better(); every thread gets the result.
@@ -207,17 +208,24 @@ constexpr int kPartWords = 4 + 2 * kCuts;
 // column 4 vecs + vt of an aligned row's remainder.
 struct PartCols {
   bool vec;
-  int vecs;      // vectors (or columns) in the strided part
+  uint32_t vecs; // vectors (or columns) in the strided part
   int steps;     // steps that any lane of the part takes
   int list0;     // first entry of the part's list in the row's buffer
+  int first;     // the part's first vector
+  // The lane's vector of a step (past 2^31 where the last step of such a row is not full).
+  __device__ __forceinline__ uint32_t at(int lane, int step) const {
+    return static_cast<uint32_t>(first + lane) + static_cast<uint32_t>(kSampleThreads) * step;
+  }
 };
 
 __device__ __forceinline__ PartCols part_cols(const float* row, int cols, int q) {
   PartCols p;
   p.vec = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
-  p.vecs = p.vec ? cols >> 2 : cols;
-  p.steps = max(0, ceil_div(p.vecs - 64 * q, kSampleThreads));
-  const int full = p.vecs / kSampleThreads, rem = p.vecs % kSampleThreads;
+  const int vecs = p.vec ? cols >> 2 : cols;
+  p.vecs = vecs;
+  p.first = 64 * q;
+  p.steps = vecs > p.first ? (vecs - p.first - 1) / kSampleThreads + 1 : 0;
+  const int full = vecs / kSampleThreads, rem = vecs % kSampleThreads;
   const int before = 64 * full * q + min(rem, 64 * q);  // vectors of the parts before
   p.list0 = p.vec ? 4 * before + (q > 0 ? cols & 3 : 0) : before;
   return p;
@@ -252,7 +260,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_max_kernel(
     float4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int i = 64 * q + lane + kSampleThreads * (m0 + wave + 4 * u);
+      const uint32_t i = pc.at(lane, m0 + wave + 4 * u);
       if (i < pc.vecs) {
         if (pc.vec) {
           v[u] = reinterpret_cast<const float4*>(row)[i];
@@ -263,7 +271,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_max_kernel(
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int i = 64 * q + lane + kSampleThreads * (m0 + wave + 4 * u);
+      const uint32_t i = pc.at(lane, m0 + wave + 4 * u);
       if (i < pc.vecs) {
         if (pc.vec) {
           take(v[u].x, 4 * i);
@@ -276,7 +284,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_max_kernel(
       }
     }
   }
-  if (pc.vec && q == 0 && wave == 0 && 4 * pc.vecs + lane < cols)
+  if (pc.vec && q == 0 && wave == 0 && 4 * pc.vecs + lane < static_cast<uint32_t>(cols))
     take(row[4 * pc.vecs + lane], 4 * pc.vecs + lane);
   for (int mask = 1; mask < 64; mask <<= 1) {
     const float ov = lane_xor(bv, mask);
@@ -405,7 +413,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
     float4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int i = 64 * q + lane + kSampleThreads * (m0 + wave + 4 * u);
+      const uint32_t i = pc.at(lane, m0 + wave + 4 * u);
       v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       if (i < pc.vecs) {
         if (pc.vec) {
@@ -420,7 +428,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
     for (int u = 0; u < U; ++u) {
       const int m = m0 + wave + 4 * u;
       if (m < pc.steps) {  // uniform
-        const int i = 64 * q + lane + kSampleThreads * m;
+        const uint32_t i = pc.at(lane, m);
         const bool ok = i < pc.vecs;
         float4 e = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         e.x = exp_of(v[u].x, ok);
@@ -441,7 +449,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
         for (int m = 0; m < 8; ++m) e[m] = s_e[min(m1 + m, n - 1)][lane];
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
-          if (m1 + m < n && 64 * q + lane + kSampleThreads * (m0 + m1 + m) < pc.vecs) {
+          if (m1 + m < n && pc.at(lane, m0 + m1 + m) < pc.vecs) {
             part += e[m].x;
             if (pc.vec) {
               part += e[m].y;
@@ -455,8 +463,8 @@ __global__ void __launch_bounds__(kPartThreads) sample_sum_kernel(
     __syncthreads();
   }
   if (wave == 0 && pc.vec && q == 0 && (cols & 3) != 0) {
-    const int c = 4 * pc.vecs + lane;
-    const bool ok = c < cols;
+    const uint32_t c = 4 * pc.vecs + lane;
+    const bool ok = c < static_cast<uint32_t>(cols);
     const float e = exp_of(ok ? row[c] : 0.0f, ok);
     if (ok) part += e;
   }
@@ -512,7 +520,7 @@ __device__ __forceinline__ void draw_all(const float* __restrict__ row, int cols
     float4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int i = 64 * q + lane + kSampleThreads * (m0 + wave + 4 * u);
+      const uint32_t i = pc.at(lane, m0 + wave + 4 * u);
       v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       if (i < pc.vecs) {
         if (pc.vec) {
@@ -525,7 +533,7 @@ __device__ __forceinline__ void draw_all(const float* __restrict__ row, int cols
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int i = 64 * q + lane + kSampleThreads * (m0 + wave + 4 * u);
+      const uint32_t i = pc.at(lane, m0 + wave + 4 * u);
       if (i < pc.vecs) {
         if (pc.vec) {
           take(v[u].x, 4 * i);
@@ -538,7 +546,7 @@ __device__ __forceinline__ void draw_all(const float* __restrict__ row, int cols
       }
     }
   }
-  if (pc.vec && q == 0 && wave == 0 && 4 * pc.vecs + lane < cols)
+  if (pc.vec && q == 0 && wave == 0 && 4 * pc.vecs + lane < static_cast<uint32_t>(cols))
     take(row[4 * pc.vecs + lane], 4 * pc.vecs + lane);
   for (int mask = 1; mask < 64; mask <<= 1) {
     const float ov = lane_xor(bv, mask);
@@ -629,7 +637,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_list_kernel(
     float4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int i = 64 * q + lane + kSampleThreads * (m0 + wave + 4 * u);
+      const uint32_t i = pc.at(lane, m0 + wave + 4 * u);
       v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       if (i < pc.vecs) {
         if (pc.vec) {
@@ -644,7 +652,7 @@ __global__ void __launch_bounds__(kPartThreads) sample_list_kernel(
     for (int u = 0; u < U; ++u) {
       const int m = m0 + wave + 4 * u;
       if (m < pc.steps) {  // uniform
-        const int i = 64 * q + lane + kSampleThreads * m;
+        const uint32_t i = pc.at(lane, m);
         const bool ok = i < pc.vecs;
         if (pc.vec) {
           take(v[u].x, 4 * i, ok);
@@ -658,8 +666,9 @@ __global__ void __launch_bounds__(kPartThreads) sample_list_kernel(
     }
   }
   if (wave == 0 && pc.vec && q == 0 && (cols & 3) != 0) {
-    const int c = 4 * pc.vecs + lane;
-    take(c < cols ? row[c] : 0.0f, c, c < cols);
+    const uint32_t c = 4 * pc.vecs + lane;
+    const bool ok = c < static_cast<uint32_t>(cols);
+    take(ok ? row[c] : 0.0f, c, ok);
   }
 }
 

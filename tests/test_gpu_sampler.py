@@ -232,3 +232,28 @@ def test_few_rows_draw_as_among_many(vocab):
     got = _sample(logits.cuda()[at.cuda()], t[at], k[at], p[at], (17 * ids + 5)[at],
                   (31 * ids)[at])
     assert torch.equal(got, want[at])
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+def test_row_of_the_largest_width(offset):
+    """2^31 - 1 columns, where a step past the row's end passes 2^31: greedy, top-k and unlimited
+    draws and the argmax of a row that is, and one that is not, 16-byte aligned."""
+    from sid.kernels.ops import argmax_rows, sample_rows
+    v = (1 << 31) - 1
+    print(f"sampler columns={v} offset={offset}", flush=True)
+    buf = torch.full((v + 8,), -30.0, device="cuda")
+    row = buf[offset:offset + v].view(1, v)
+    buf[:offset] = buf[offset + v:] = 9.0  # (outside the row)
+    at = [0, 65, v // 2, v - 1000, v - 2, v - 1]
+    for c, x in zip(at, (1.0, 2.0, 1.5, 2.5, 2.0, 3.0)):
+        buf[offset + c] = x
+    assert argmax_rows(row).tolist() == [v - 1]
+    one = lambda x, dt=torch.int64: torch.tensor([x], dtype=dt, device="cuda")
+    draw = lambda t, k, p, s: sample_rows(row, one(t, torch.float32), one(k), one(p, torch.float32),
+                                          one(s), one(3)).item()
+    assert draw(0.0, -1, 1.0, 1) == v - 1
+    assert draw(0.5, 1, 1.0, 1) == v - 1
+    assert draw(0.5, -1, 0.1, 1) == v - 1
+    got = {draw(5.0, 6, 1.0, s) for s in range(4)}
+    assert got <= set(at) and len(got) > 1
+    assert draw(0.25, -1, 1.0, 5) in at  # (elsewhere at most log 1e-10 + 16.7)
