@@ -469,12 +469,12 @@ __device__ __forceinline__ int swz(int key) { return (key & 3) | (((key >> 3) & 
 // Lane l's 16 bytes at its address -> LDS byte lds + 16 l.
 __device__ __forceinline__ void dma16(const void* src, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds)
-               : "memory");
+               : "memory", "m0");
 }
 __device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off),
                "s"(base), "s"(lds)
-               : "memory");
+               : "memory", "m0");
 }
 
 constexpr int kTileBytes = BN * D * 2;  // one K or V tile

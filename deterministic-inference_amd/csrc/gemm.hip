@@ -458,7 +458,7 @@ __device__ __forceinline__ void dma16(uint32_t voff, u32x4_v srd, uint32_t soff,
   asm volatile(
       "s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff),
       "s"(srd), "s"(soff), "s"(lds)
-      : "memory");
+      : "memory", "m0");
 }
 
 // All but this wave's N newest loads have landed, its LDS reads are done, and every wave of
