@@ -932,6 +932,20 @@ void launch_tile(const void* x, int64_t ldx, const void* w, int64_t m, int64_t n
 // round trips of few workgroups, which smaller tiles spread over more CUs: 777 x 1024 x 3072
 // 20.7 (128 x 128) vs 11.6 us (64 x 64), 2048 x 1024 x 2048 15.1 (128 x 128) vs 12.7 (128 x
 // 64), 8420 x 1024 x 2048 50.5 (256 x 128, a second round for 8 tiles) vs 43.7 (128 x 128).
+int tile_shape(int64_t m, int64_t n) {
+  const int64_t cus = cu_count();
+  auto tiles = [&](int tm, int tn) { return ((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
+  auto rounds = [&](int64_t t, int64_t slots) { return (t + slots - 1) / slots; };
+  const int64_t t64 = tiles(64, 64);
+  const int64_t cost[4] = {970 * rounds(tiles(256, 128), cus), 500 * rounds(tiles(128, 128), cus),
+                           330 * rounds(tiles(128, 64), cus),
+                           t64 <= cus ? 210 : 380 * rounds(t64, 2 * cus)};
+  int best = 0;
+  for (int i = 1; i < 4; ++i)
+    if (cost[i] < cost[best]) best = i;
+  return best;
+}
+
 template <int EPI>
 void launch_tiles(const void* x, int64_t ldx, const void* w, int64_t m, int64_t n, int64_t k,
                   const TileOut& out, hipStream_t s) {
@@ -939,17 +953,7 @@ void launch_tiles(const void* x, int64_t ldx, const void* w, int64_t m, int64_t 
     // 128-column tiles: the candidate grouping of the lm_head epilogues
     launch_tile<4, 2, 2, 4, 4, 2, 1, EPI>(x, ldx, w, m, n, k, out, s);
   } else {
-    const int64_t cus = cu_count();
-    auto tiles = [&](int tm, int tn) { return ((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
-    auto rounds = [&](int64_t t, int64_t slots) { return (t + slots - 1) / slots; };
-    const int64_t t64 = tiles(64, 64);
-    const int64_t cost[4] = {970 * rounds(tiles(256, 128), cus), 500 * rounds(tiles(128, 128), cus),
-                             330 * rounds(tiles(128, 64), cus),
-                             t64 <= cus ? 210 : 380 * rounds(t64, 2 * cus)};
-    int best = 0;
-    for (int i = 1; i < 4; ++i)
-      if (cost[i] < cost[best]) best = i;
-    switch (best) {
+    switch (tile_shape(m, n)) {
       case 0: launch_tile<4, 2, 4, 4, 3, 2, 1, EPI>(x, ldx, w, m, n, k, out, s); break;
       case 1: launch_tile<4, 2, 2, 4, 4, 2, 1, EPI>(x, ldx, w, m, n, k, out, s); break;
       case 2: launch_tile<4, 2, 2, 2, 5, 2, 1, EPI>(x, ldx, w, m, n, k, out, s); break;
@@ -1838,6 +1842,11 @@ __global__ void __launch_bounds__(NCH * 64) linear_silu_kernel(const bf16_t* __r
 }  // namespace sid
 
 using namespace sid;
+
+extern "C" int sid_linear_tile(int64_t m, int64_t n) {
+  constexpr int shape[4] = {256 << 16 | 128, 128 << 16 | 128, 128 << 16 | 64, 64 << 16 | 64};
+  return m > 0 && n > 0 ? shape[tile_shape(m, n)] : 0;
+}
 
 extern "C" int sid_linear(const void* x, int64_t ldx, const void* w, const void* bias, void* y,
                           int64_t m, int64_t n, int64_t k, int out_fp32, void* stream) {

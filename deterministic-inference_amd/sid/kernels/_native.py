@@ -61,7 +61,7 @@ EXPORTED = ("sid_last_error", "sid_abi_version", "sid_extend_attention_workspace
             "sid_linear_argmax_workspace_bytes", "sid_sample_workspace_bytes",
             "sid_qwen3_extend_workspace_bytes", "sid_qwen3_extend_forward",
             "sid_flash_decode_noalloc_scratch_bytes", "sid_linear_sample_workspace_bytes",
-            "sid_extend_attention_query_rows", *_SIGNATURES)
+            "sid_extend_attention_query_rows", "sid_linear_tile", *_SIGNATURES)
 ABI_VERSION = 22
 
 
@@ -106,6 +106,8 @@ class NativeLib:
         self.lib.sid_extend_attention_workspace_bytes.argtypes = [_i32, _i64, _i32, _i32, _i32, _i32]
         self.lib.sid_extend_attention_query_rows.restype = ctypes.c_int
         self.lib.sid_extend_attention_query_rows.argtypes = [_i32, _i64, _i32, _i32]
+        self.lib.sid_linear_tile.restype = ctypes.c_int
+        self.lib.sid_linear_tile.argtypes = [_i64, _i64]
         self.lib.sid_linear_argmax_workspace_bytes.restype = ctypes.c_int64
         self.lib.sid_linear_argmax_workspace_bytes.argtypes = [_i64]
         self.lib.sid_sample_workspace_bytes.restype = ctypes.c_int64

@@ -256,6 +256,10 @@ int sid_rope_apply(void* q, void* k, const int64_t* positions, const float* cos_
 int sid_linear(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t m,
                int64_t n, int64_t k, int out_fp32, void* stream);
 
+/* Rows << 16 | columns of the output tiles with which sid_linear and the SwiGLU form (N = 2
+ * inter) cover [M, N] on the current device: a speed choice, the results are the same. */
+int sid_linear_tile(int64_t m, int64_t n);
+
 /*
  * Split-K form of sid_linear without bias: partials fp32 [K/256][M][N] gets
  * the sum of each 256-wide K chunk (accumulated exactly as in sid_linear).

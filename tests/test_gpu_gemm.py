@@ -146,20 +146,34 @@ def test_linear_argmax_ties_and_nan(m):
 
 
 
+def _folded(x, w):
+    """x w^T in fp32 by the split-K kernel, its chunks folded in order."""
+    from sid.kernels.jit import load_ext
+    part = torch.empty(x.shape[1] // 256, x.shape[0], w.shape[0], device="cuda",
+                       dtype=torch.float32)
+    load_ext().linear_partials(x, w, part)
+    fold = part[0].clone()
+    for c in part[1:]:
+        fold += c
+    return fold
+
+
 @pytest.mark.parametrize("m,n,k", [(256, 1024, 1024), (300, 1024, 2048), (1000, 6144, 1024),
                                    (2048, 4096, 1024), (777, 192, 512), (4100, 1024, 3072)])
-def test_tiled_large_m_bitwise_matches_row_group_kernel(m, n, k):
-    """M >= 64 takes the LDS-tiled MFMA kernel (128 x 128 or 128 x 64 tiles); its bits
-    equal the 64-row-group kernel's on row slices of fewer than 64 rows, and its own on a
-    129-row slice, with bias, both output dtypes, ragged M and N tails."""
+def test_tiled_large_m_bitwise_matches_folded_chunks(m, n, k):
+    """The tile kernel's bits equal the split-K chunks folded in order (rows in groups of 64
+    there), and its own on slices of fewer and more than 64 rows, which take other tiles,
+    with bias, both output dtypes, ragged M and N tails."""
     from sid.kernels.matmul_persistent import linear
     torch.manual_seed(m + n)
     print(f"m={m} n={n} k={k}", flush=True)
     x = torch.randn(m, k, device="cuda", dtype=torch.bfloat16)
     w = (torch.randn(n, k, device="cuda") * 0.05).to(torch.bfloat16)
     b = torch.randn(n, device="cuda", dtype=torch.bfloat16)
+    fold = _folded(x, w)
     for bias in (None, b):
         full = linear(x, w, bias)
+        assert torch.equal(full, (fold if bias is None else fold + b.float()).to(torch.bfloat16))
         for lo, hi in ((0, 63), (m - 33, m), (m // 2, m // 2 + 129)):
             assert torch.equal(full[lo:hi], linear(x[lo:hi].contiguous(), w, bias)), (lo, hi)
     f32 = linear(x, w, out_fp32=True)
@@ -168,38 +182,41 @@ def test_tiled_large_m_bitwise_matches_row_group_kernel(m, n, k):
     torch.testing.assert_close(f32[:64].cpu(), ref, atol=3e-2, rtol=2e-2)
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (1, 64, 256),        # one row
-    (33, 128, 1024),     # one tile of rows, the first SwiGLU rows on tiles
-    (63, 1024, 3072),    # a row short of a tile
-    (64, 64, 256),       # one 64 x 64 tile, one chunk (the shortest K pipeline)
-    (300, 1024, 2048),   # 64 x 64 tiles, ragged rows
-    (1030, 1088, 768),   # 128 x 64 tiles, ragged rows
-    (1025, 3200, 256),   # 128 x 128 tiles, one row in the last ones, one chunk
-    (1500, 4032, 512),   # 256 x 128 tiles, half a tile of columns left
-    (4353, 8128, 256),   # 256 x 128 tiles, several rounds of the grid, one chunk
+@pytest.mark.parametrize("m,n,k,tile", [
+    (1, 64, 256, (64, 64)),          # one row
+    (33, 128, 1024, (64, 64)),       # one tile of rows, the first SwiGLU rows on tiles
+    (63, 1024, 3072, (64, 64)),      # a row short of a tile
+    (64, 64, 256, (64, 64)),         # one tile, one chunk (the shortest K pipeline)
+    (300, 1024, 2048, (64, 64)),     # ragged rows
+    (1030, 1088, 768, (128, 64)),    # ragged rows
+    (1025, 3200, 256, (128, 128)),   # one row in the last tiles, one chunk
+    (4353, 8128, 256, (128, 128)),   # several rounds of the grid, one chunk
+    (1500, 4032, 512, (256, 128)),   # half a tile of columns left
+    (8190, 6144, 256, (256, 128)),   # several rounds of the grid, ragged rows, one chunk
+    (8190, 6144, 1024, (256, 128)),  # the same, four chunks
+    (4999, 6080, 768, (256, 128)),   # several rounds, ragged rows and columns
 ])
-def test_tile_kernel_edges_bitwise(m, n, k):
-    """The pipelined tile GEMM in each tile shape, at the edges of tiles and of the K pipeline:
-    bits of the split-K kernel's chunks folded in order, for bf16 and fp32 outputs with and
-    without bias, from rows inside a wider matrix, into an output that is only 2- (4-) byte
-    aligned, with the rows after the output untouched; and the SwiGLU form against
-    sid_linear + sid_silu_mul."""
+def test_tile_kernel_edges_bitwise(m, n, k, tile):
+    """The pipelined tile GEMM in each tile shape, at the edges of tiles, of the K pipeline and
+    of the grid's rounds (a tile's first loads run while the tile before it is stored): bits of
+    the split-K kernel's chunks folded in order, for bf16 and fp32 outputs with and without
+    bias, from rows inside a wider matrix, into an output that is only 2- (4-) byte aligned,
+    with the rows after the output untouched; and the SwiGLU form against sid_silu_mul of the
+    folded chunks."""
     from sid.kernels.jit import load_ext
-    from sid.kernels.matmul_persistent import linear, linear_silu_mul
+    from sid.kernels.matmul_persistent import linear_silu_mul
     from sid.kernels.ops import silu_mul
     ext = load_ext()
     torch.manual_seed(m + n + k)
     print(f"tile edges m={m} n={n} k={k}", flush=True)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        got = ext.lib.sid_linear_tile(m, n)
+        assert (got >> 16, got & 0xffff) == tile
     big = torch.randn(m, k + 64, device="cuda", dtype=torch.bfloat16)
     x = big[:, :k]
     w = (torch.randn(n, k, device="cuda") * 0.05).to(torch.bfloat16)
     b = torch.randn(n, device="cuda", dtype=torch.bfloat16)
-    part = torch.empty(k // 256, m, n, device="cuda", dtype=torch.float32)
-    ext.linear_partials(x, w, part)
-    fold = part[0].clone()
-    for c in range(1, k // 256):
-        fold += part[c]
+    fold = _folded(x, w)
     for bias in (None, b):
         ref = (fold if bias is None else fold + b.float()).to(torch.bfloat16)
         for fp32 in (False, True):
@@ -210,14 +227,10 @@ def test_tile_kernel_edges_bitwise(m, n, k):
                 ext.linear(x, w, bias, y, fp32)
                 assert torch.equal(y, ref.to(dt)), (bias is not None, fp32, off)
                 assert (buf[off + m * n:] == 7.0).all()
-    if k == 256:
-        return
-    x = x.contiguous()
-    if k != 1024:  # the SwiGLU entry takes K = 1024
+    if (n // 2) % 64 == 0:  # the SwiGLU entry takes K = 1024
         x = torch.randn(m, 1024, device="cuda", dtype=torch.bfloat16)
         w = (torch.randn(n, 1024, device="cuda") * 0.05).to(torch.bfloat16)
-    if (n // 2) % 64 == 0:
-        assert torch.equal(linear_silu_mul(x, w), silu_mul(linear(x, w)))
+        assert torch.equal(linear_silu_mul(x, w), silu_mul(_folded(x, w).to(torch.bfloat16)))
 
 
 @pytest.mark.parametrize("m,ldx", [(2, 1 << 23), (65, 1 << 25)])

@@ -130,10 +130,10 @@ def test_positions_draws_equal_oracle_and_respect_top_p():
 
 @pytest.mark.parametrize("vocab", [151936, 20001, 1023, 7, 1])
 def test_list_and_full_paths_vs_exact_oracle(vocab):
-    """Rows whose cut lies in the listed columns (near the maximum), at the list's capacity
-    (8192 columns) and its threshold, beyond it (flat rows, nuclei wider than the list), with
-    long runs of equal keys at the cut, and with masked (-inf) columns; an odd vocabulary
-    puts rows off 16-byte alignment, tiny ones leave most parts of a row empty."""
+    """Rows whose cut lies in the listed columns (near the maximum), beyond them (flat rows,
+    nuclei wider than the list), with long runs of equal keys at the cut, and with masked
+    (-inf) columns; an odd vocabulary puts rows off 16-byte alignment, tiny ones leave most
+    parts of a row empty."""
     g = torch.Generator().manual_seed(vocab + 1)
     n = lambda *s: torch.randn(*s, generator=g)
     rows, cfg = [], []
@@ -149,14 +149,14 @@ def test_list_and_full_paths_vs_exact_oracle(vocab):
     flat = n(vocab) * 0.3
     for t, k, p in ((1.0, -1, 0.9), (1.0, 40, 1.0), (2.0, 3, 0.2), (1.0, -1, 0.0)):
         add(flat, t, k, p)
-    for near in (8191, 8192, 8193):  # columns within the list's threshold, the rest far below
+    for near in (8191, 8192, 8193):  # that many equal columns, the rest far below
         row = torch.full((vocab,), -40.0)
         row[torch.randperm(vocab, generator=g)[:near]] = 0.0
         row[vocab // 2] = 1.0
         add(row, 1.0, 500, 1.0)
         add(row, 1.0, -1, 0.5)
-        add(row, 1.0, 9000, 1.0)  # reaches past the list
-    edge = torch.full((vocab,), -9.703125)  # exp(-9.703125) just above 2^-14
+        add(row, 1.0, 9000, 1.0)  # reaches past the equal columns
+    edge = torch.full((vocab,), -9.703125)  # every other column equal
     edge[0] = 0.0
     add(edge, 1.0, 10, 1.0)
     add(edge - 0.0625 * torch.arange(vocab).clamp(max=3), 1.0, 3, 1.0)
@@ -257,3 +257,61 @@ def test_row_of_the_largest_width(offset):
     got = {draw(5.0, 6, 1.0, s) for s in range(4)}
     assert got <= set(at) and len(got) > 1
     assert draw(0.25, -1, 1.0, 5) in at  # (elsewhere at most log 1e-10 + 16.7)
+
+
+def _check_both_forms(rows, cfg):
+    """Few rows (four launches where they are long), and the same rows among 160 (one launch)."""
+    m = len(rows)
+    logits = torch.stack(rows)
+    t, k, p = (list(x) for x in zip(*cfg))
+    seeds, pos = [17 * i + 5 for i in range(m)], [31 * i for i in range(m)]
+    got = _check(logits, t, k, p, seeds, pos)
+    at = torch.arange(160) % m
+    many = _sample(logits.cuda()[at.cuda()], *(torch.tensor(x)[at] for x in (t, k, p, seeds, pos)))
+    assert torch.equal(many, got[at])
+
+
+LIST_CAP, CUTS = 16384, (6, 9, 12, 15, 18, 21)  # kListCap and -log2 of kCutMin of sample.hip
+
+
+@pytest.mark.parametrize("vocab", [151936, 40001])
+def test_list_capacity_vs_exact_oracle(vocab):
+    """Exactly the list's capacity of columns above a threshold, one less and one more, with
+    limits at, before and past the last of them."""
+    print(f"list capacity vocab={vocab}", flush=True)
+    g = torch.Generator().manual_seed(vocab)
+    rows, cfg = [], []
+    for near in (LIST_CAP - 1, LIST_CAP, LIST_CAP + 1):
+        row = torch.full((vocab,), -60.0)
+        at = torch.randperm(vocab, generator=g)[:near]
+        row[at] = -2.0 * torch.rand(near, generator=g)  # exp of at least 2^-3
+        row[at[0]] = 1.0
+        for k, p in ((near, 1.0), (near - 1, 1.0), (near + 1, 1.0), (-1, 0.5), (-1, 0.9999)):
+            rows.append(row)
+            cfg.append((1.0, k, p))
+    _check_both_forms(rows, cfg)
+
+
+@pytest.mark.parametrize("vocab", [151936, 40001])
+def test_list_thresholds_vs_exact_oracle(vocab):
+    """For each threshold 60 columns just above it and 60 just below (apart by more than the
+    roundings of x / T and of the exponential, about 4 ulp), the limit at the last one above,
+    at the first below and between; with temperatures and maxima that stretch the logits'
+    bound by which the list's candidates are picked."""
+    print(f"list thresholds vocab={vocab}", flush=True)
+    g = torch.Generator().manual_seed(vocab + 1)
+    rows, cfg = [], []
+    for i, cut in enumerate(CUTS):
+        for t, top in ((1.0, 0.0), (0.3, 300.0), (7.0, -2000.0), (1.7, 40.0))[i % 2::2]:
+            gap = 4e-6 + 8 * 2.0 ** -24 * abs(top) / t
+            row = torch.full((vocab,), top - 60.0 * t)
+            at = torch.randperm(vocab, generator=g)[:121]
+            row[at[0]] = top
+            row[at[1:61]] = top + t * (-cut * math.log(2) + gap)
+            row[at[61:]] = top + t * (-cut * math.log(2) - gap)
+            mass = 60 * 2.0 ** -cut  # of each group, the maximum's being 1
+            for k, p in ((61, 1.0), (62, 1.0), (31, 1.0), (-1, (1 + 0.5 * mass) / (1 + 2 * mass)),
+                         (-1, (1 + 1.5 * mass) / (1 + 2 * mass))):
+                rows.append(row)
+                cfg.append((t, k, p))
+    _check_both_forms(rows, cfg)
