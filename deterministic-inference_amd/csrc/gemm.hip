@@ -428,8 +428,8 @@ struct SampleIn {
 //
 // LDS: a stage's rows are 128 bytes (64 bf16) without padding, 16-byte piece p of row q at
 // p ^ ((q >> 1) & 7): the DMA writes whole 1 KB runs (the permutation is on the global side,
-// inside one 128-byte line) and the fragment reads are conflict-free (SQ_LDS_BANK_CONFLICT
-// 0). Rows past M or N are dropped by the buffer range check (zeros); their outputs are not
+// inside one 128-byte line) and the fragment reads are conflict-free (SQ_LDS_BANK_CONFLICT 512
+// a 256 x 128 tile at any K, from the store staging alone). Rows past M or N are dropped by the buffer range check (zeros); their outputs are not
 // stored. Weights are the MFMA's A operand, so a lane holds four consecutive columns of one
 // row and a tile is stored through LDS as whole 128-byte lines.
 //
@@ -2002,8 +2002,8 @@ static void launch_sample_mbs(const bf16_t* x, int64_t ldx, const void* w, int m
 // The streaming sampler reads the weights once per 64-row group; above this many rows (or
 // when asked) the tiled GEMM with the sampler epilogue reads them once per 128-row tile
 // (candidate groups: 128-column tiles instead of streaming waves). Measured at T = 0.7,
-// 151936 x 1024, graph-timed (streaming vs tiled, us): 1 row 73 vs 91, 64 rows 108 vs
-// 119, 96 rows 181 vs 132, 128 rows 199 vs 137, 192 rows 291 vs 216, 256 rows 375 vs 238.
+// 151936 x 1024, graph-timed (streaming vs tiled, us): 1 row 75 vs 97, 64 rows 112 vs
+// 128, 96 rows 183 vs 144, 128 rows 199 vs 147, 200 rows 354 vs 234, 256 rows 378 vs 250.
 constexpr int64_t kStreamSampleMaxM = 64;
 
 extern "C" int sid_linear_sample(const void* x, int64_t ldx, const void* w, int64_t m, int64_t n,

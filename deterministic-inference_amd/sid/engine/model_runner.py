@@ -135,8 +135,8 @@ class ModelRunner:
           * batch_invariant decode batches: the engine's one choice (_invariant_fused), with
             the streaming grouping at every size;
           * other decode batches: by speed, grouping by row count (T = 0.7, graph-timed:
-            1 row 80 vs 178 us for logits + sampler kernel, 64: 120 vs 205, 128: 158 vs 231,
-            256: 284 vs 329); dvr commits only the verifier's tokens, nondet is free."""
+            1 row 78 vs 102 us for logits + sampler, 64: 111 vs 139, 128: 143 vs 200,
+            256: 247 vs 258); dvr commits only the verifier's tokens, nondet is free."""
         if not fb.untruncated:
             return False
         if fb.mode in (ForwardMode.PREFILL, ForwardMode.VERIFY):

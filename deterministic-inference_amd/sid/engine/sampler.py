@@ -1,6 +1,6 @@
 """Row-independent sampler shared by decode and the DVR verifier (sid/engine/sampler.py).
 
-Every row is drawn by one HIP kernel (`sid_sample_rows`): greedy rows (temperature 0) take
+Every row is drawn by one HIP call (`sid_sample_rows`): greedy rows (temperature 0) take
 the argmax with first-index ties; stochastic rows take softmax(logits / T), the top-k /
 top-p truncation of the reference (sid/engine/sampler.py:45-58, with the mass before a
 rank summed exactly in fixed point), and the seeded Gumbel-max draw whose noise is a hash

@@ -194,6 +194,9 @@ def test_prefill_kernel_edges_bitwise(specs, slots):
     longest = max(e for _, e in specs)
     tiles = -(-longest // 32)
     assert len(specs) * HKV * tiles >= 512  # the full batch does not fan out
+    from sid.kernels.jit import load_ext
+    rows = load_ext().lib.sid_extend_attention_query_rows(len(specs), q.shape[0], HKV, longest)
+    assert rows == (64 if longest == 1024 else 32)
     full = _fwd(q, kb, vb, qo, kvp, idx, longest, SCALE)
     assert torch.isinf(full[int(qo[1]) - 1, :, 3]).all()  # (infinite, not NaN: inf / l)
     for b in range(len(specs)):
