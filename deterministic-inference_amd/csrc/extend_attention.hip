@@ -489,14 +489,15 @@ __global__ void __launch_bounds__(NW * 64, NW / 2) extend_prefill_kernel(
     bf16_t* __restrict__ o) {
   extern __shared__ __align__(1024) char lds[];  // [2][K tile, V tile]
   constexpr int ROWS = 8 * NW;  // query positions of the workgroup
-  const int b = blockIdx.x;
-  if (b >= batch) return;  // (the grid's padding)
+  // (The grid's padding returns with the empty tiles: a branch of its own before the loads of
+  // the indices cost every workgroup their latency, 512 x 16 tokens 35.1 -> 35.7 us.)
+  const int b = min(static_cast<int>(blockIdx.x), batch - 1);
   const int h_kv = blockIdx.y;
   // Late query tiles walk the most keys: dispatch them first.
   const int mtile = mtiles - 1 - static_cast<int>(blockIdx.z);
   const int q_start = qo_indptr[b];
   const int extend_len = qo_indptr[b + 1] - q_start;
-  if (mtile * ROWS >= extend_len) return;
+  if (mtile * ROWS >= extend_len || static_cast<int>(blockIdx.x) >= batch) return;
   const int kv_start = kv_indptr[b];
   const int kv_len = kv_indptr[b + 1] - kv_start;
   const int prefix = kv_len - extend_len;
